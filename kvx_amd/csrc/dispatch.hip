@@ -313,104 +313,170 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
   return grid_fits(*grid, t->threads);
 }
 
-// Tiled block write plan (write_tiles_kernel): at least bs tokens,
-// power-of-two bs (<= one wave) and cache row bytes, dense blocks of which
-// at least one is not row-major, 16-byte aligned block addresses, io rows
-// aligned to the tile op's source chunk, and (quantizing) heads a whole
-// number of 8-element chunks, so that every chunk has one scale.
-// kWriteTileBytes: cache bytes per tensor of one tile of a copying write;
-// kQuantTileBytes the same for the FP8 quantizing write (whose
-// io rows are 2-4x its cache bytes).  On MI355X (c3 shapes, inputs not
-// cache-resident) 8 KiB measured 1.5-3% faster than 16 KiB for copies, and
-// 4-5% faster than 32 or 64 KiB; the quantizing write is 4-8% faster with
-// 16 KiB; 4 KiB is 25-30% slower for both.  Tiles are 0-5% faster than
-// staging whole blocks of K and V in one workgroup (x-packed / HND), 5x for
-// the token-innermost value cache.
+// Tiled write plan (write_tiles_kernel): dense blocks of which at least one
+// is not row-major, 16-byte aligned block addresses, cache rows of whole
+// 16-byte chunks, io rows aligned to the tile op's source chunk, and
+// (quantizing) heads a whole number of 8-element chunks, so that every chunk
+// has one scale.  The constants by measurement on MI355X (same process,
+// medians, us per launch):
+//
+// kWriteTileBytes: cache bytes per tensor of one workgroup, and
+// kWriteLdsCopyBytes those of a copy through LDS (76800 tokens of 8 x 128
+// bf16 in 16-token blocks, 8 -> 16 KiB: x-packed 120.3 -> 118.7, vLLM's pair
+// 121.6 -> 118.3; HND, direct, 118.2 -> 119.6).  A quantizing workgroup of 16
+// KiB would take more than kTileLoads chunks per lane.  Batches that make
+// fewer than kWriteTileWorkgroups of them per tensor (decode) halve them down
+// to kWriteTileMin, so that the rows spread over the CUs (64 decode tokens,
+// 8 -> 2 -> 1 KiB: x-packed 4.33 -> 3.63 -> 3.45, vLLM's pair 8.35 -> 6.07 ->
+// 5.30; 4000 tokens unchanged).
 constexpr int64_t kWriteTileBytes = 8192;
-constexpr int64_t kQuantTileBytes = 16384;
+constexpr int64_t kWriteLdsCopyBytes = 16384;
+constexpr int64_t kWriteTileMin = 1024;
+constexpr int64_t kWriteTileWorkgroups = 512;
+// Tokens per workgroup of staged and narrow tensors, at most: 16 store half
+// lines of narrow runs (vLLM's pair, 64-token blocks, 19200 tokens: 74
+// against 33) and x-packed chunks that start inside blocks took 38 against
+// 27; 64 leave a wave no lanes for the rows that follow (narrow: 174).
+constexpr int64_t kWriteTileRows = 32;
+// Bytes of a narrow run that one workgroup stores whole, at most.
+constexpr int64_t kWriteAlignBytes = 64;
+// Bytes per row of a direct tensor's workgroup, at most: whole rows of 2 KiB
+// measured 112 and 108 for HND 32-token blocks (76800 tokens, chunks starting
+// inside blocks and on them), 512 bytes 117 and 117.
+constexpr int64_t kWriteDirectWidth = 2048;
+
+// The divisor of `row` that is a multiple of `unit` and at most `target`,
+// the widest of whole 128-byte lines first; the narrowest one when all are
+// wider than target.
+int64_t tile_width(int64_t row, int64_t unit, int64_t target) {
+  const int64_t n = row / unit;
+  if ((n & (n - 1)) == 0) {
+    int64_t w = unit;
+    while (w < row && w * 2 <= target) w *= 2;
+    return w;
+  }
+  int64_t best = -1, line = -1;
+  for (int64_t k = 1; k <= row / unit; ++k) {
+    if ((row / unit) % k != 0) continue;
+    const int64_t w = unit * k;
+    if (w > target && best > 0) break;
+    best = w;
+    if (w % 128 == 0) line = w;
+    if (w > target) break;
+  }
+  return line > 0 ? line : best;
+}
+
 bool plan_write_tiles(const WritePlan &p, int cs, int is, WriteTileArgs *wt, int64_t *grid,
-                      uint32_t *lds_bytes) {
+                      int32_t *threads, uint32_t *lds_bytes) {
   const int64_t bs = p.block_size;
   const int64_t H = p.heads;
   const int64_t D = p.head_dim;
-  const int64_t row_cache = H * D * cs;
-  const int bs_log2 = log2_exact(bs);
-  if (bs_log2 < 0 || bs > kWave || p.num_tokens < bs) return false;
-  if (row_cache < 16) return false;
-  const int src_chunk = p.conv == kConvQuant ? 8 * is : 16;
-  if (p.conv == kConvQuant && D % 8 != 0) return false;
+  const int64_t row = H * D * cs;  // cache bytes
+  const bool quant = p.conv == kConvQuant;
+  const int chunk = quant ? 8 : 16;  // cache bytes of the op's chunk
+  const int src_chunk = chunk / cs * is;
+  if (row % 16 != 0 || (quant && D % 8 != 0)) return false;
   const Geom *g[2] = {&p.gk, &p.gv};
   const void *src[2] = {p.src_k, p.src_v};
-  const void *dst[2] = {p.dst_k, p.dst_v};
-  bool transposed = false, odd_run = false;
-  int64_t min_tw = 16;
-  int64_t unit = 16;  // a tile width holds whole runs and 16-byte chunks
+  void *dst[2] = {p.dst_k, p.dst_v};
+  const ScaleRef sc[2] = {p.k_scale, p.v_scale};
+  int64_t run_elems[2];
   for (int i = 0; i < 2; ++i) {
-    const int64_t w = dense_run_elems(*g[i], bs, H, D);
-    if (w < 0) return false;
-    wt->run_log2[i] = w == H * D ? -1 : log2_exact(w * cs);
-    wt->run_bytes[i] = 0;
-    wt->run_magic[i] = 0;
-    if (w != H * D) {
-      if (wt->run_log2[i] < 0) {
-        // runs that are not a power of two: 16-byte pieces, one run each
-        if ((w * cs) % 16 != 0) return false;
-        wt->run_log2[i] = kRunOdd;
-        wt->run_bytes[i] = (int32_t)(w * cs);
-        // unstage_tile_odd divides region offsets (< 64 KiB) by the run
-        wt->run_magic[i] = magic_for(w * cs);
-        odd_run = true;
-      }
-      transposed = true;
-      if (w * cs > min_tw) min_tw = w * cs;
-      unit = unit / gcd64(unit, w * cs) * (w * cs);
-    }
+    run_elems[i] = dense_run_elems(*g[i], bs, H, D);
+    if (run_elems[i] < 0) return false;
+  }
+  // row-major pairs: the flat kernel
+  if (run_elems[0] == H * D && run_elems[1] == H * D) return false;
+  int64_t base_tile = kWriteTileBytes;
+  while (base_tile > kWriteTileMin && p.num_tokens * row / base_tile < kWriteTileWorkgroups)
+    base_tile /= 2;
+  int64_t wgs = 0, need = 0, lds = 0;
+  for (int i = 0; i < 2; ++i) {
+    const int64_t w = run_elems[i];
+    const int64_t run = w * cs;
+    if (run % 16 != 0 && (run > 8 || (run & (run - 1)) != 0)) return false;
     if ((reinterpret_cast<uintptr_t>(dst[i]) | (uintptr_t)(g[i]->s_block * cs)) % 16 != 0)
       return false;
     if ((reinterpret_cast<uintptr_t>(src[i]) | (uintptr_t)(H * D * is)) % src_chunk != 0)
       return false;
+    WriteTileTensor &t = wt->t[i];
+    t.kind = w == H * D || run % 128 == 0 ? kTileDirect : run >= 16 ? kTileStaged : kTileNarrow;
+    int64_t tile = base_tile;
+    if (t.kind != kTileDirect && !quant && tile == kWriteTileBytes &&
+        p.num_tokens * row / kWriteLdsCopyBytes >= kWriteTileWorkgroups)
+      tile = kWriteLdsCopyBytes;
+    // a tile holds whole 16-byte pieces and whole runs
+    const int64_t unit = w == H * D || run < 16 ? 16 : run;
+    const int64_t target = t.kind == kTileDirect
+                               ? (tile < kWriteDirectWidth ? tile : kWriteDirectWidth)
+                               : (tile / kWriteTileRows < 128 ? 128 : tile / kWriteTileRows);
+    const int64_t tw = tile_width(row, unit, target);
+    int rows_log2 = 0;
+    const int64_t cap = t.kind == kTileDirect ? kWave : kWriteTileRows;
+    while ((2 << rows_log2) <= cap && (tw << (rows_log2 + 1)) <= tile) ++rows_log2;
+    const int64_t cpr = tw / chunk;
+    if ((cpr << rows_log2) > need) need = cpr << rows_log2;
+    t.src = static_cast<const char *>(src[i]);
+    t.dst = static_cast<char *>(dst[i]);
+    t.s_block = g[i]->s_block * cs;
+    t.s_run = bs * run;
+    t.sc = sc[i];
+    t.run = (int32_t)run;
+    t.run_log2 = log2_exact(run);
+    t.rows = 1 << rows_log2;
+    t.rows_log2 = rows_log2;
+    t.tw = (int32_t)tw;
+    t.tiles = (int32_t)(row / tw);
+    t.cpr = (int32_t)cpr;
+    // exact: u * cpr <= 2^32 for u < 4 * kBlockThreads and cpr of that order
+    t.cpr_magic = cpr > 1 ? magic_for(cpr) : 0;
+    t.pitch = (int32_t)(tw + kTilePad);
+    // narrow runs: units of 16 bytes (8 bytes of 1-byte runs in 8-token
+    // blocks) that blocks hold a whole number of
+    t.seg = 1;
+    if (t.kind == kTileNarrow) {
+      const int64_t seg = 16 / run;
+      if (bs % seg == 0) t.seg = (int32_t)seg;
+      else if (run == 1 && bs % 8 == 0) t.seg = 8;
+    }
+    // aligned slots of one line (narrow: sector) of a run, as far as one
+    // wave's lanes hold the slots of the rows and of those that follow them
+    t.align = 1;
+    if (t.kind == kTileStaged || t.seg > 1) {
+      const int64_t whole = t.kind == kTileStaged ? 128 : kWriteAlignBytes;
+      while (t.align * run < whole && bs % (t.align * 2) == 0 && t.align * 2 <= t.rows &&
+             t.rows + t.align * 2 <= kWave)
+        t.align *= 2;
+      if (t.align < t.seg) t.align = 1;
+    }
+    const int64_t n = (p.num_tokens + t.rows - 1) / t.rows * t.tiles;
+    if (n > 0x7FFFFFFF) return false;
+    t.workgroups = (uint32_t)n;
+    if (n > wgs) wgs = n;
+    const int64_t lrows = t.rows + (t.align > 1 ? t.align : 0);
+    const int64_t l = t.kind == kTileDirect ? 0 : lrows * (t.pitch + 12);
+    if (l > lds) lds = l;
   }
-  if (!transposed) return false;
-  const int64_t tile_bytes =
-      p.conv == kConvQuant ? kQuantTileBytes : kWriteTileBytes;
-  // as in plan_tiles: a power-of-two tile width that divides the row, and
-  // a full copy tile for a row that is not a power of two (c3's size into
-  // HND caches of 6 x 128 or 12 x 64 bf16 heads: 0.527 of peak against 0.43
-  // per token); otherwise a tile of whole runs (odd_tile_width): at c3's
-  // size, 3 heads of 128 measured 0.61 of peak against 0.11 per token for
-  // an x-packed K, 0.58 against 0.055 for vLLM's K / V pair and 0.68 against
-  // 0.50 for HND; HND 8 x 80 0.61 against 0.50, 8 x 96 0.60 against 0.57
-  int64_t tw = row_cache & -row_cache;
-  if (odd_run || tw < min_tw ||
-      ((row_cache & (row_cache - 1)) != 0 && tw * bs < kWriteTileBytes)) {
-    tw = odd_tile_width(row_cache, unit, bs, tile_bytes);
-    if (tw < 0) return false;
-  } else {
-    while (tw * bs > tile_bytes && tw / 2 >= min_tw) tw /= 2;
-  }
-  const int64_t pitch = tw + kTilePad;
-  if (bs * pitch > 64 * 1024) return false;
-  wt->tiles = (int32_t)(row_cache / tw);
-  wt->tw = (int32_t)tw;
-  wt->tw_log2 = log2_exact(tw);
-  // phase 1 chunks per row (Op::kDst cache bytes each: 16, or 8 FP8 bytes);
-  // div_magic is exact since u * cpr < bs * tw * tw <= 2^16 * tw
-  wt->cpr = (int32_t)(tw / (p.conv == kConvQuant ? 8 : 16));
-  wt->cpr_magic = wt->tw_log2 < 0 ? magic_for(wt->cpr) : 0;
-  wt->pitch = (int32_t)pitch;
-  // about one thread per kTileBytesPerThread bytes of tile, as for
-  // the gather: small tiles (one KV head) in smaller workgroups.  On MI355X
-  // (c3's bytes in one-head rows) vLLM's pair 61.3 -> 53.4 us, x-packed K
-  // and V 58.6 -> 53.1 us; c3's own 8 KiB tiles unchanged.
-  wt->threads = kBlockThreads;
-  while (wt->threads > 64 && tw * bs < (int64_t)wt->threads * kTileBytesPerThread)
-    wt->threads /= 2;
-  wt->bs_log2 = bs_log2;
+  // about one thread per kTileBytesPerThread bytes of tile, and at most
+  // kTileLoads chunks each
+  int64_t nt = kBlockThreads;
+  while (nt > kWave && (nt / 2) * kTileBytesPerThread >= need * chunk && (nt / 2) * kTileLoads >= need)
+    nt /= 2;
+  if (need > nt * kTileLoads || lds > 64 * 1024) return false;
+  wt->slots = p.slots;
+  wt->num_tokens = p.num_tokens;
+  wt->row_bytes = H * D * is;
+  wt->slot_is64 = p.slot_is64;
+  wt->block_size = p.block_size;
+  wt->bs_log2 = log2_exact(bs);
+  wt->num_blocks = p.num_blocks;
+  wt->head_dim = p.head_dim;
   wt->cache_es_log2 = log2_exact(cs);
-  wt->io_es_log2 = log2_exact(is);
-  *grid = (p.num_tokens + bs - 1) / bs * wt->tiles;
-  *lds_bytes = (uint32_t)(bs * pitch);
-  return grid_fits(*grid, wt->threads);
+  *grid = wgs;
+  *threads = (int32_t)nt;
+  *lds_bytes = (uint32_t)lds;
+  return grid_fits(*grid, (int)nt);
 }
 
 }  // namespace
@@ -464,7 +530,7 @@ kvx_status_t enqueue_write(const WritePlan &p, void *stream) {
   // loop: on MI355X a 2048-workgroup cap made c3-sized NHD prefill writes
   // 2-4% slower (8% with blocks in ascending order).
   wl.grid = (int)(want < 65536 ? want : 65536);
-  wl.tiles = plan_write_tiles(p, cs, is, &wl.wt, &wl.tile_grid, &wl.tile_lds);
+  wl.tiles = plan_write_tiles(p, cs, is, &wl.wt, &wl.tile_grid, &wl.tile_threads, &wl.tile_lds);
   // write_flat_kernel: K and V rows hold H * D consecutive elements.  A
   // chunk count that is not a power of two (576-element MLA rows: 72) finds
   // a chunk's token by multiply-high, exact while the largest flat index

@@ -632,653 +632,346 @@ __global__ __launch_bounds__(kFlatThreads) void write_flat_kernel(WriteArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Block write (prefill into a layout that is not row-major in the block).
+// Tiled write into dense blocks that are not both row-major.
 //
-// When the `bs` consecutive tokens of a group fill one cache block in order
-// (slot = b * bs + o for o = 0..bs-1, the usual prefill pattern), the
-// group's source rows are one contiguous io region and each cache tensor's
-// destination is one contiguous block region, only permuted.
-// write_tiles_kernel moves such groups through LDS so that both the io
-// reads and the cache writes are coalesced 16-byte accesses; groups that do
-// not fill a block take the per-token path.
-
-// A run of a group: tokens [t0 + tok, t0 + tok + hi - lo) hold the slots
-// block * bs + lo .. block * bs + hi - 1, in order.
-struct GroupRun {
-  int64_t block;
-  int32_t lo;
-  int32_t hi;
-  int32_t tok;
-  int32_t pad_;
+// A workgroup takes `rows` consecutive tokens (at most one wave's lanes) and
+// `tw` cache bytes of each of their rows, of one tensor (blockIdx.y: K 0,
+// V 1).  Every row goes to its own slot, whatever the slots are: prefill
+// chunks in order or starting inside blocks, decode batches, -1.  The loads
+// of a lane's row chunks are issued first; each wave loads the slots itself,
+// one per lane, so that the two latencies overlap, and shares them by
+// shuffles.  How a tensor's rows reach its blocks depends on the bytes of a
+// row that lie together in the block, its run:
+//   direct   runs of whole 128-byte lines (NHD, most HND): a lane stores the
+//            chunks it loaded;
+//   staged   shorter runs of 16 bytes and more (x-packed): through LDS rows
+//            (pitch tw + 16 bytes), then 16-byte pieces with the token
+//            fastest over the lanes, so that consecutive slots are stored as
+//            consecutive pieces;
+//   narrow   runs below 16 bytes (token axis innermost): through LDS rows;
+//            tokens whose slots fill an aligned unit of `seg` = 16 / run
+//            slots in order are stored together, a lane reading one column
+//            of `seg` rows, and every other token run by run.
+// Staged and narrow tensors: tokens of consecutive slots inside `align`
+// aligned slots all belong to the workgroup in whose tokens they start, which
+// also loads the rows that follow its own, so that no cache line (narrow:
+// 64-byte sector) of a chunk that starts inside a block is stored in parts by
+// two workgroups.
+// HBM bounds it (and, for batches below a few hundred KB, the latency of one
+// load and one store); what costs is not the transposition but lines stored
+// in parts and loads in series.  A kernel that told whole blocks apart from
+// other groups by a run analysis, with two barriers and a second load of
+// slots and rows, and that took blocks of at most 64 tokens, measured on
+// MI355X (same process, medians, us per launch, 19200 tokens of 8 x 128 bf16
+// in 16 chunks starting inside blocks, before -> this kernel): HND 16-token
+// blocks 33 -> 25, x-packed 16 / 64 / 128 tokens 33 / 41 / 208 -> 28 / 28 /
+// 28, vLLM's pair 16 / 64 / 128 tokens 36 / 121 / 946 -> 29 / 33 / 34; 200
+// decode tokens HND 4.1 -> 3.2, vLLM's pair 8.7 -> 7.0.  Chunks that start on
+// blocks were within 1% from 19200 to 76800 tokens.  Without `align`, the
+// latter's x-packed write starting inside blocks took 138 us against 120,
+// and vLLM's pair at 19200 tokens 101 against 29.
+struct WriteTileTensor {
+  const char *src;
+  char *dst;
+  int64_t s_block;      // bytes
+  int64_t s_run;        // bytes between a row's consecutive runs
+  ScaleRef sc;          // quantizing ops only
+  int32_t kind;         // kTileDirect, kTileStaged or kTileNarrow
+  int32_t run;          // bytes of a run (a whole row when row-major)
+  int32_t run_log2;     // log2(run), or -1
+  int32_t rows;         // tokens per workgroup, a power of two <= 64
+  int32_t rows_log2;
+  int32_t tw;           // cache bytes per row of a workgroup
+  int32_t tiles;        // workgroups per `rows` tokens: row bytes / tw
+  int32_t cpr;          // chunks per tile row
+  uint32_t cpr_magic;   // div_magic's m for cpr, 0 when cpr is 1
+  int32_t pitch;        // LDS row pitch, bytes
+  int32_t seg;          // narrow: slots of a unit
+  int32_t align;        // 1: a workgroup stores its own tokens only
+  uint32_t workgroups;
 };
+constexpr int32_t kTileDirect = 0;
+constexpr int32_t kTileStaged = 1;
+constexpr int32_t kTileNarrow = 2;
 
-// Runs a group's tokens may form and still be written through LDS: a prefill
-// chunk of bs consecutive positions covers the end of one block and the
-// start of the next.
-constexpr int kMaxRuns = 2;
-
-// Wave 0 splits tokens [t0, t0 + bs) into runs of consecutive offsets of one
-// block and writes them to runs[] (LDS); *nruns = their count, or 0 when a
-// token's slot is < 0 or past the blocks or there are more than kMaxRuns
-// runs (the group is then written token by token).  Read after the caller's
-// __syncthreads().
-__device__ __forceinline__ void group_runs(const WriteArgs &a, int64_t t0, int bs_log2,
-                                           GroupRun *runs, int32_t *nruns) {
-  const int tid = (int)threadIdx.x;
-  if (tid >= kWave) return;
-  const int lane = tid;
-  const int64_t left = a.num_tokens - t0;
-  const int n = left < (1 << bs_log2) ? (int)left : (1 << bs_log2);
-  int64_t slot = -1;
-  if (lane < n) slot = load_index(a.slots, t0 + lane, a.slot_is64);
-  const int64_t blk = slot >> bs_log2;
-  const int32_t off = (int32_t)(slot & ((1 << bs_log2) - 1));
-  const bool ok = lane >= n || (slot >= 0 && blk < a.num_blocks);
-  const int64_t prev = (int64_t)(((uint64_t)(uint32_t)__shfl_up((int)(slot >> 32), 1) << 32) |
-                                 (uint32_t)__shfl_up((int)slot, 1));
-  const bool start = lane < n && (lane == 0 || off == 0 || slot != prev + 1);
-  const uint64_t bad = __ballot(!ok);
-  const uint64_t starts = __ballot(start);
-  const int count = __popcll(starts);
-  const bool take = bad == 0 && count <= kMaxRuns;
-  if (lane == 0) *nruns = take ? count : 0;
-  if (take && start) {
-    const uint64_t later = lane == kWave - 1 ? 0ull : starts & (~0ull << (lane + 1));
-    const int end = later ? __ffsll((long long)later) - 1 : n;
-    GroupRun r;
-    r.block = blk;
-    r.lo = off;
-    r.hi = off + (end - lane);
-    r.tok = lane;
-    r.pad_ = 0;
-    runs[__popcll(starts & ((1ull << lane) - 1ull))] = r;
-  }
-}
-
-// Run ownership for block sizes up to 32 (2 * bs slots fit one wave), for
-// tensors whose blocks are not row-major.  A run here is a maximal stretch
-// of tokens whose slots are valid, lie in one block and follow each other
-// (slot = previous slot + 1).  The workgroups of group [t0, t0 + bs) own
-// the runs that START in it; such a run ends before t0 + 2 * bs - 1, since
-// it holds at most bs tokens.  Every token then has exactly one owner, and
-// a prefill chunk that starts inside a block has each of its blocks written
-// whole by one workgroup instead of split between two, whose writes would
-// share cache lines (or 16-byte chunks, stored piece by piece).  On MI355X
-// (c3's size, x-packed K, chunks starting k = 1, 11 or 15 tokens into a
-// block) splitting the x-packed blocks measured 79 us against 55-62 us for
-// owned runs; only k = 8, whose halves are whole 128-byte lines, gained.
-// A whole block in order (write_tile_block's case) is one run starting at
-// t0 either way.
-//
-// Wave 0 loads the slots of tokens t0 - 1 .. t0 + 2 * bs - 2, one per lane,
-// and writes the owned runs to runs[] (LDS); *nruns = their count, or 0
-// when an owned token's slot is < 0 or past the blocks or there are more
-// than kMaxRuns runs (the owned tokens are then written token by token).
-// own[0], own[1]: the owned tokens, [t0 + own[0], t0 + own[1]).  Read after
-// the caller's __syncthreads().
-__device__ __forceinline__ void owned_runs(const WriteArgs &a, int64_t t0, int bs_log2,
-                                           GroupRun *runs, int32_t *nruns, int32_t *own) {
-  const int lane = (int)threadIdx.x;
-  if (lane >= kWave) return;
-  const int bs = 1 << bs_log2;
-  const int64_t t = t0 - 1 + lane;  // lane 0: the token before the group
-  const bool in = lane < 2 * bs && t >= 0 && t < a.num_tokens;
-  int64_t slot = -1;
-  if (in) slot = load_index(a.slots, t, a.slot_is64);
-  const int64_t blk = slot >> bs_log2;
-  const int32_t off = (int32_t)(slot & (bs - 1));
-  const bool ok = in && slot >= 0 && blk < a.num_blocks;
-  const int64_t prev = (int64_t)(((uint64_t)(uint32_t)__shfl_up((int)(slot >> 32), 1) << 32) |
-                                 (uint32_t)__shfl_up((int)slot, 1));
-  const uint64_t oks = __ballot(ok);
-  const uint64_t ins = __ballot(in);
-  const bool prev_ok = lane > 0 && ((oks >> (lane - 1)) & 1ull);
-  // Lanes without a token count as starts: they bound the last run.
-  const bool start = !in || !ok || !prev_ok || off == 0 || slot != prev + 1;
-  const uint64_t starts = __ballot(start);
-  const uint64_t group = ((1ull << bs) - 1ull) << 1;  // lanes of tokens t0 .. t0 + bs - 1
-  const uint64_t mine = starts & group & ins;
-  if (mine == 0) {
-    // The group's tokens all continue a run that starts before t0.
-    if (lane == 0) {
-      *nruns = 0;
-      own[0] = 0;
-      own[1] = 0;
-    }
-    return;
-  }
-  const int first = __ffsll((long long)mine) - 1;
-  const int last = 63 - __clzll((long long)mine);
-  const uint64_t after = last >= 63 ? 0ull : starts & (~0ull << (last + 1));
-  const int end = after ? __ffsll((long long)after) - 1 : kWave;  // exclusive lane
-  const uint64_t owned = (end >= kWave ? ~0ull : ((1ull << end) - 1ull)) & (~0ull << first);
-  const bool bad = (~oks & owned & ins) != 0;
-  const int count = __popcll(mine);
-  const bool take = !bad && count <= kMaxRuns;
-  if (lane == 0) {
-    *nruns = take ? count : 0;
-    own[0] = first - 1;
-    own[1] = end - 1;
-  }
-  if (take && ((mine >> lane) & 1ull)) {
-    const uint64_t later = lane >= 63 ? 0ull : starts & (~0ull << (lane + 1));
-    const int e = later ? __ffsll((long long)later) - 1 : kWave;
-    GroupRun r;
-    r.block = blk;
-    r.lo = off;
-    r.hi = off + (e - lane);
-    r.tok = lane - 1;
-    r.pad_ = 0;
-    runs[__popcll(mine & ((1ull << lane) - 1ull))] = r;
-  }
-}
-
-// Per-token write of one tensor (V when v, else K) for the tokens
-// [t0, t0 + n) of a group that does not fill a block, shared by `nwaves`
-// waves: this workgroup's wave w is wave wave0 + w of them and takes tokens
-// wave0 + w, wave0 + w + nwaves, ...
-template <class Op, bool IDX>
-__device__ __forceinline__ void write_group_tokens(const WriteArgs &a, int64_t t0, int n, bool v,
-                                                   float uniform, int wave0, int nwaves) {
-  const int lane = (int)(threadIdx.x & (kWave - 1));
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-  const GeomBytes &g = v ? a.gv : a.gk;
-  const ScaleRef &sr = v ? a.vsc : a.ksc;
-  const char *io = v ? a.src_v : a.src_k;
-  char *cache = v ? a.dst_v : a.dst_k;
-  for (int o = wave0 + wave; o < n; o += nwaves) {
-    const int64_t t = t0 + o;
-    if (t >= a.num_tokens) break;
-    const int64_t slot = load_index(a.slots, t, a.slot_is64);
-    if (slot < 0) continue;
-    int64_t b, off;
-    split_slot(slot, a.block_size, b, off);
-    if (b >= a.num_blocks) continue;
-    const char *src = io + t * a.row_bytes;
-    char *dst = cache + b * g.s_block + off * g.s_off;
-    for (int c = lane; c < a.nchunks; c += kWave) {
-      const uint32_t e = (uint32_t)c * (uint32_t)a.chunk_elems;
-      float sc = uniform;
-      if constexpr (Op::kScaled && IDX) sc = scale_at(sr, uniform, b, e, (uint32_t)a.head_dim);
-      st<Op::kDst, kWriteNtStore>(dst + chunk_off(g, e, (uint32_t)a.head_dim),
-                                  Op::apply(ld<Op::kSrc>(src + (int64_t)c * Op::kSrc), sc));
-    }
-  }
-}
-
-// Tiled block write: the inverse of gather_tiles_kernel (below).  A group
-// is `bs` consecutive tokens; when their slots form at most kMaxRuns runs of
-// consecutive offsets of one block each (a whole block in order, or a
-// prefill chunk that starts inside a block), a workgroup takes tile `tile`
-// (tw cache bytes of every row) of one tensor (blockIdx.y: K 0, V 1) and,
-// run by run:
-//   phase 1  reads the tile's columns of the run's source rows, applies the
-//            chunk op (copy, or FP8 quantization with the scale of the
-//            run's block and the chunk's head)
-//            and stores the cache bytes in LDS rows (pitch tw + 16 bytes);
-//   phase 2  assembles each 16-byte chunk of the block region
-//            [tile * tw * bs, (tile + 1) * tw * bs) from its run pieces and
-//            stores it; chunks holding rows outside the run store those
-//            rows' pieces only.
-// A row-major tensor copies its rows straight through.  Any other group is
-// written token by token, each tensor's tokens spread over the waves of
-// that tensor's `tiles` workgroups of the group.
 struct WriteTileArgs {
-  int32_t tiles;          // tiles per block: cache row bytes / tw
-  int32_t tw;             // tile width, cache bytes per row
-  int32_t tw_log2;        // log2(tw), or -1 when tw is not a power of two
-  int32_t cpr;            // tw_log2 < 0: phase-1 chunks per tile row
-  uint32_t cpr_magic;     // tw_log2 < 0: div_magic's m for cpr
-  int32_t pitch;          // LDS row pitch, bytes
-  int32_t threads;        // workgroup size (64-256, by tile bytes)
-  int32_t bs_log2;
-  int32_t run_log2[2];    // K, V: log2 bytes of a per-token run; -1 row-major;
-                          // kRunOdd: run_bytes, a multiple of 16 bytes
-  int32_t run_bytes[2];
-  uint32_t run_magic[2];  // kRunOdd: div_magic's m for run_bytes
-  int32_t cache_es_log2;  // log2 cache element bytes
-  int32_t io_es_log2;     // log2 io element bytes
+  WriteTileTensor t[2];
+  const void *slots;
+  int64_t num_tokens;
+  int64_t row_bytes;    // io bytes of a row
+  int32_t slot_is64;
+  int32_t block_size;
+  int32_t bs_log2;      // log2(block_size), or -1
+  int32_t num_blocks;
+  int32_t head_dim;
+  int32_t cache_es_log2;
 };
 
-// Row and chunk of tile chunk u (cpr chunks per tile row): shifts when the
-// tile width is a power of two, a multiply-high division otherwise (ODD).
-template <bool ODD>
-__device__ __forceinline__ int32_t tile_row(int32_t u, int32_t cpr_log2, const WriteTileArgs &wt) {
-  if constexpr (ODD) return (int32_t)div_magic((uint32_t)u, wt.cpr_magic);
-  else return u >> cpr_log2;
-}
-template <bool ODD>
-__device__ __forceinline__ int32_t tile_col(int32_t u, int32_t row, int32_t cpr_log2,
-                                            const WriteTileArgs &wt) {
-  if constexpr (ODD) return u - row * wt.cpr;
-  else return u & ((1 << cpr_log2) - 1);
+__device__ __forceinline__ int64_t shfl64(int64_t x, int lane) {
+  return (int64_t)(((uint64_t)(uint32_t)__shfl((int)(x >> 32), lane) << 32) |
+                   (uint32_t)__shfl((int)x, lane));
 }
 
-// Piece k (PIECE bytes) of a 16-byte chunk, read from p into x (x's other
-// pieces untouched; x starts zeroed for PIECE < 4).
-template <int PIECE>
-__device__ __forceinline__ void get_piece(const char *p, Raw<16> &x, int k) {
-  if constexpr (PIECE == 16) {
-    x = ld<16>(p);
-  } else if constexpr (PIECE == 8) {
-    const Raw<8> y = ld<8>(p);
-    x.w[2 * k] = y.w[0];
-    x.w[2 * k + 1] = y.w[1];
-  } else if constexpr (PIECE == 4) {
-    x.w[k] = ld<4>(p).w[0];
-  } else if constexpr (PIECE == 2) {
-    put16(x, k, ld<2>(p).w[0]);
+// x / d by div_magic, or x for d = 1 (m = 0).
+__device__ __forceinline__ uint32_t div_or_same(uint32_t x, uint32_t m) {
+  return m ? div_magic(x, m) : x;
+}
+
+// Narrow runs: the tile's full units, `count` of them, tab[i] the first row
+// of unit i: a lane takes one run of the SEG rows of one unit.
+template <int W, int SEG>
+__device__ __forceinline__ void store_units(const WriteTileTensor &t, const char *lds,
+                                            const int64_t *off, const int32_t *tab, int32_t count,
+                                            char *dst) {
+  const int32_t cols = t.tw / W;
+  // units fastest over the lanes when they are a power of two: the units of a
+  // block lie side by side in each of its runs
+  const bool p2 = (count & (count - 1)) == 0;
+  const int32_t lg = 31 - __clz(count);
+  for (int32_t u = (int32_t)threadIdx.x; u < count * cols; u += (int32_t)blockDim.x) {
+    const int32_t i = p2 ? u & (count - 1) : u / cols;
+    const int32_t c = p2 ? u >> lg : u - i * cols;
+    const int32_t r = tab[i];
+    const char *p = lds + r * t.pitch + c * W;
+    Raw<SEG * W> y;
+    if constexpr (W < 4) {
+#pragma unroll
+      for (int k = 0; k < Raw<SEG * W>::kWords; ++k) y.w[k] = 0;
+    }
+#pragma unroll
+    for (int k = 0; k < SEG; ++k) {
+      if constexpr (W == 1) {
+        put8(y, k, ld<1>(p + k * t.pitch).w[0]);
+      } else if constexpr (W == 2) {
+        put16(y, k, ld<2>(p + k * t.pitch).w[0]);
+      } else {
+        const Raw<W> x = ld<W>(p + k * t.pitch);
+#pragma unroll
+        for (int j = 0; j < W / 4; ++j) y.w[k * (W / 4) + j] = x.w[j];
+      }
+    }
+    st<SEG * W, kWriteNtStore>(dst + off[r] + (int64_t)c * t.s_run, y);
+  }
+}
+
+// Every other token of the tile (tab[0 .. count)), run by run.
+template <int W>
+__device__ __forceinline__ void store_tokens(const WriteTileTensor &t, const char *lds,
+                                             const int64_t *off, const int32_t *tab,
+                                             int32_t count, char *dst) {
+  const int32_t cols = t.tw / W;
+  const bool p2 = (cols & (cols - 1)) == 0;
+  const int32_t lg = 31 - __clz(cols);
+#pragma unroll 4
+  for (int32_t u = (int32_t)threadIdx.x; u < count * cols; u += (int32_t)blockDim.x) {
+    const int32_t i = p2 ? u >> lg : u / cols;
+    const int32_t c = u - i * cols;
+    const int32_t r = tab[i];
+    st<W, kWriteNtStore>(dst + off[r] + (int64_t)c * t.s_run, ld<W>(lds + r * t.pitch + c * W));
+  }
+}
+
+// Op moves kDst cache bytes a chunk.  IDX: per-head / per-block scales.
+// NARROW: one of the tensors is narrow.
+template <class Op, bool IDX, bool NARROW>
+__global__ __launch_bounds__(kBlockThreads) void write_tiles_kernel(WriteTileArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const WriteTileTensor &t = a.t[blockIdx.y];
+  if (blockIdx.x >= t.workgroups) return;
+  const uint32_t gu = blockIdx.x / (uint32_t)t.tiles;
+  const uint32_t tile = blockIdx.x - gu * (uint32_t)t.tiles;
+  const int64_t t0 = (int64_t)gu << t.rows_log2;
+  const int32_t left = a.num_tokens - t0 < t.rows ? (int32_t)(a.num_tokens - t0) : t.rows;
+  const int32_t tid = (int32_t)threadIdx.x;
+  const int32_t lane = tid & (kWave - 1);
+  const int32_t nt = (int32_t)blockDim.x;
+
+  // Lane l holds the slot of row l - lane0 of the tile (narrow: from the row
+  // before it to the rows that may follow it).
+  const int32_t lane0 = t.align > 1 ? 1 : 0;
+  const int64_t ts = t0 + lane - lane0;
+  int64_t slot = -1;
+  if (ts >= 0 && ts < a.num_tokens && lane < t.rows + lane0 * t.align)
+    slot = load_index(a.slots, ts, a.slot_is64);
+  // chunk u is chunk u % cpr of row u / cpr
+  const int32_t total = left * t.cpr;
+  const char *src = t.src + t0 * a.row_bytes + (int64_t)tile * t.cpr * Op::kSrc;
+  Raw<Op::kSrc> x[kTileLoads];
+  int32_t row[kTileLoads];
+#pragma unroll
+  for (int k = 0; k < kTileLoads; ++k) {
+    const int32_t u = tid + k * nt;
+    row[k] = (int32_t)div_or_same((uint32_t)u, t.cpr_magic);
+    if (u < total)
+      x[k] = ld<Op::kSrc, kWriteNtLoad>(src + row[k] * a.row_bytes +
+                                        (int64_t)(u - row[k] * t.cpr) * Op::kSrc);
+  }
+  float uniform = 1.0f;
+  if constexpr (Op::kScaled) uniform = t.sc.p[0];
+
+  int64_t b, o;
+  if (a.bs_log2 >= 0) {
+    b = slot >> a.bs_log2;
+    o = slot & (a.block_size - 1);
   } else {
-    put8(x, k, ld<1>(p).w[0]);
+    split_slot(slot < 0 ? 0 : slot, a.block_size, b, o);
   }
-}
+  const bool ok = slot >= 0 && b < a.num_blocks;
+  // of the row's first run in its block; -1: the row is skipped
+  const int64_t off = ok ? b * t.s_block + o * t.run : -1;
+  const int32_t blk = ok ? (int32_t)b : 0;
+  const int32_t c0 = (int32_t)tile * t.tw;  // the tile's first cache byte of a row
 
-// Phase 2 of the tiled write: LDS rows -> region (nbytes = tw * bs cache
-// bytes, 16-byte aligned), rows [lo, hi) only.  PIECE = min(run bytes, 16).
-// A 16-byte chunk whose pieces all belong to rows in [lo, hi) is stored
-// whole; a chunk that mixes rows (runs shorter than 16 bytes, partial
-// blocks) stores the pieces of its rows in range one by one.  FULL: every
-// row is in range (a whole block), and the row tests are compiled out.
-template <int PIECE, bool FULL>
-__device__ __forceinline__ void unstage_tile(char *region, const char *lds, int32_t nbytes,
-                                             int32_t run_log2, int32_t bs_log2, int32_t pitch,
-                                             int32_t lo, int32_t hi) {
-  const int32_t bsm = (1 << bs_log2) - 1;
-  const int32_t runm = (1 << run_log2) - 1;
-  const int32_t kStep = (int32_t)blockDim.x * 16;
-  for (int32_t m0 = (int32_t)threadIdx.x * 16; m0 < nbytes; m0 += kTileLoads * kStep) {
-    Raw<16> x[kTileLoads];
-    bool whole[kTileLoads];
+  // Scale of chunk u, in row r: of the row's block and the chunk's head.
+  auto scale_of_chunk = [&](int32_t u, int32_t r, bool in) {
+    float sc = uniform;
+    if constexpr (Op::kScaled && IDX) {
+      const int32_t rb = __shfl(blk, (r + lane0) & (kWave - 1));
+      const uint32_t e = (uint32_t)(c0 + (u - r * t.cpr) * Op::kDst) >> a.cache_es_log2;
+      if (in) sc = scale_at(t.sc, uniform, rb, e, (uint32_t)a.head_dim);
+    }
+    return sc;
+  };
+
+  if (t.kind == kTileDirect) {
 #pragma unroll
-    for (int u = 0; u < kTileLoads; ++u) {
-      const int32_t m = m0 + u * kStep;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x[u].w[i] = 0;
-      whole[u] = m < nbytes;
-      if (m < nbytes) {
-#pragma unroll
-        for (int k = 0; k < 16 / PIECE; ++k) {
-          const int32_t mm = m + k * PIECE;
-          const int32_t o = (mm >> run_log2) & bsm;
-          const int32_t ar = mm >> (run_log2 + bs_log2);
-          const char *p = lds + o * pitch + (ar << run_log2) + (mm & runm);
-          if (FULL || (o >= lo && o < hi)) {
-            get_piece<PIECE>(p, x[u], k);
-          } else {
-            whole[u] = false;
-          }
-        }
+    for (int k = 0; k < kTileLoads; ++k) {
+      if (k * nt >= total) break;  // the same for every lane
+      const int32_t u = tid + k * nt;
+      const int64_t ro = shfl64(off, row[k] & (kWave - 1));
+      const float sc = scale_of_chunk(u, row[k], u < total);
+      if (u < total && ro >= 0) {
+        const uint32_t c = (uint32_t)(c0 + (u - row[k] * t.cpr) * Op::kDst);
+        const uint32_t q = t.run_log2 >= 0 ? c >> t.run_log2 : c / (uint32_t)t.run;
+        st<Op::kDst, kWriteNtStore>(
+            t.dst + ro + (int64_t)q * t.s_run + (c - q * (uint32_t)t.run), Op::apply(x[k], sc));
       }
-    }
-#pragma unroll
-    for (int u = 0; u < kTileLoads; ++u) {
-      const int32_t m = m0 + u * kStep;
-      if (whole[u]) {
-        st<16, kWriteNtStore>(region + m, x[u]);
-      } else if (!FULL && m < nbytes) {
-#pragma unroll
-        for (int k = 0; k < 16 / PIECE; ++k) {
-          const int32_t mm = m + k * PIECE;
-          const int32_t o = (mm >> run_log2) & bsm;
-          if (o >= lo && o < hi) {
-            const int32_t ar = mm >> (run_log2 + bs_log2);
-            st<PIECE, kWriteNtStore>(region + mm,
-                                     ld<PIECE>(lds + o * pitch + (ar << run_log2) + (mm & runm)));
-          }
-        }
-      }
-    }
-  }
-}
-
-// Phase 2 for runs of `run` bytes, a multiple of 16 but not a power of two:
-// every 16-byte chunk lies inside one run of one row, and is stored whole
-// when that row is in [lo, hi).
-template <bool FULL>
-__device__ __forceinline__ void unstage_tile_odd(char *region, const char *lds, int32_t nbytes,
-                                                 int32_t run, uint32_t run_magic, int32_t bs_log2,
-                                                 int32_t pitch, int32_t lo, int32_t hi) {
-  const uint32_t bsm = (1u << bs_log2) - 1;
-  const int32_t kStep = (int32_t)blockDim.x * 16;
-  for (int32_t m0 = (int32_t)threadIdx.x * 16; m0 < nbytes; m0 += kTileLoads * kStep) {
-    Raw<16> x[kTileLoads];
-    bool ok[kTileLoads];
-#pragma unroll
-    for (int u = 0; u < kTileLoads; ++u) {
-      const int32_t m = m0 + u * kStep;
-      const uint32_t q = div_magic((uint32_t)m, run_magic);
-      const int32_t o = (int32_t)(q & bsm);
-      ok[u] = m < nbytes && (FULL || (o >= lo && o < hi));
-      if (ok[u]) x[u] = ld<16>(lds + o * pitch + (int32_t)(q >> bs_log2) * run + (m - (int32_t)q * run));
-    }
-#pragma unroll
-    for (int u = 0; u < kTileLoads; ++u)
-      if (ok[u]) st<16, kWriteNtStore>(region + m0 + u * kStep, x[u]);
-  }
-}
-
-// ODD: the tile width is not a power of two, as it is for every run that
-// is not (a multiple of such a run never is one), so only then can
-// run_log2 be kRunOdd.
-template <bool FULL, bool ODD>
-__device__ __forceinline__ void unstage_any(char *dst, const char *lds, int32_t region,
-                                            int32_t run_log2, const WriteTileArgs &wt,
-                                            const GroupRun &r, bool v) {
-  if constexpr (ODD) {
-    if (run_log2 == kRunOdd) {
-      unstage_tile_odd<FULL>(dst, lds, region, wt.run_bytes[v], wt.run_magic[v], wt.bs_log2,
-                             wt.pitch, r.lo, r.hi);
-      return;
-    }
-  }
-  switch (run_log2) {
-    case 0: unstage_tile<1, FULL>(dst, lds, region, 0, wt.bs_log2, wt.pitch, r.lo, r.hi); break;
-    case 1: unstage_tile<2, FULL>(dst, lds, region, 1, wt.bs_log2, wt.pitch, r.lo, r.hi); break;
-    case 2: unstage_tile<4, FULL>(dst, lds, region, 2, wt.bs_log2, wt.pitch, r.lo, r.hi); break;
-    case 3: unstage_tile<8, FULL>(dst, lds, region, 3, wt.bs_log2, wt.pitch, r.lo, r.hi); break;
-    default:
-      unstage_tile<16, FULL>(dst, lds, region, run_log2, wt.bs_log2, wt.pitch, r.lo, r.hi);
-      break;
-  }
-}
-
-// One run of a group through one tile of one tensor: rows [r.lo, r.hi) of
-// block r.block from the io rows of tokens t0 + r.tok, ...
-template <class Op, bool IDX, bool ODD>
-__device__ __forceinline__ void write_tile_run(const WriteArgs &a, const WriteTileArgs &wt,
-                                               const GroupRun &r, int64_t t0, int32_t tile,
-                                               bool v, float uniform, char *lds) {
-  const ScaleRef &sr = v ? a.vsc : a.ksc;
-  const uint32_t hd = (uint32_t)a.head_dim;
-  const char *src = (v ? a.src_v : a.src_k) + (t0 + r.tok) * a.row_bytes;
-  char *blk = v ? a.dst_v + r.block * a.gv.s_block : a.dst_k + r.block * a.gk.s_block;
-  const int32_t run_log2 = v ? wt.run_log2[1] : wt.run_log2[0];
-  const int32_t region = wt.tw << wt.bs_log2;
-  const int tid = (int)threadIdx.x;
-
-  if (run_log2 < 0) {
-    // Row-major block: rows [lo, hi) are one span of the block and of the
-    // source rows.
-    const int32_t row_bytes_c = wt.tiles * wt.tw;
-    const int32_t span_lo = r.lo * row_bytes_c;
-    const int32_t span_hi = r.hi * row_bytes_c;
-    const int32_t lo = tile * region > span_lo ? tile * region : span_lo;
-    const int32_t hi = (tile + 1) * region < span_hi ? (tile + 1) * region : span_hi;
-    const uint32_t re = (uint32_t)a.nchunks * (uint32_t)a.chunk_elems;  // H * D
-    for (int32_t m = lo + tid * Op::kDst; m < hi; m += (int32_t)blockDim.x * Op::kDst) {
-      const uint32_t e = (uint32_t)(m - span_lo) >> wt.cache_es_log2;
-      float sc = uniform;
-      if constexpr (Op::kScaled && IDX) sc = scale_in_rows(sr, uniform, r.block, e, re, hd);
-      st<Op::kDst, kWriteNtStore>(
-          blk + m, Op::apply(ld<Op::kSrc, kWriteNtLoad>(src + ((int64_t)e << wt.io_es_log2)),
-                             sc));
     }
     return;
   }
 
-  // Phase 1: chunk c of row lo + q holds the row's io elements e0 + c * G.
-  constexpr int kDstLog2 = Op::kDst == 16 ? 4 : Op::kDst == 8 ? 3 : Op::kDst == 4 ? 2
-                           : Op::kDst == 2 ? 1 : 0;
-  const int32_t cpr_log2 = wt.tw_log2 - kDstLog2;
-  const int32_t total = ODD ? (r.hi - r.lo) * wt.cpr : (r.hi - r.lo) << cpr_log2;
-  const uint32_t e0 = ((uint32_t)tile * (uint32_t)wt.tw) >> wt.cache_es_log2;
-  for (int32_t u0 = tid; u0 < total; u0 += kTileLoads * (int32_t)blockDim.x) {
-    Raw<Op::kSrc> x[kTileLoads];
-#pragma unroll
-    for (int k = 0; k < kTileLoads; ++k) {
-      const int32_t u = u0 + k * (int32_t)blockDim.x;
-      if (u < total) {
-        const int32_t row = tile_row<ODD>(u, cpr_log2, wt);
-        const int32_t col = tile_col<ODD>(u, row, cpr_log2, wt);
-        const uint32_t e = e0 + ((uint32_t)(col << kDstLog2) >> wt.cache_es_log2);
-        x[k] = ld<Op::kSrc, kWriteNtLoad>(src + (int64_t)row * a.row_bytes +
-                                          ((int64_t)e << wt.io_es_log2));
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kTileLoads; ++k) {
-      const int32_t u = u0 + k * (int32_t)blockDim.x;
-      if (u < total) {
-        const int32_t row = tile_row<ODD>(u, cpr_log2, wt);
-        const int32_t col = tile_col<ODD>(u, row, cpr_log2, wt);
-        float sc = uniform;
-        if constexpr (Op::kScaled && IDX) {
-          const uint32_t e = e0 + ((uint32_t)(col << kDstLog2) >> wt.cache_es_log2);
-          sc = scale_at(sr, uniform, r.block, e, hd);
-        }
-        st<Op::kDst>(lds + (r.lo + row) * wt.pitch + (col << kDstLog2), Op::apply(x[k], sc));
-      }
-    }
-  }
-  __syncthreads();
-  char *dst = blk + (int64_t)tile * region;
-  if (r.lo == 0 && r.hi == (1 << wt.bs_log2)) {
-    unstage_any<true, ODD>(dst, lds, region, run_log2, wt, r, v);
-  } else {
-    unstage_any<false, ODD>(dst, lds, region, run_log2, wt, r, v);
-  }
-}
-
-// Whole-block fast path of write_tiles_kernel, for the usual prefill group.
-// Aligned: the group's bs slots are block * bs + 0 .. bs - 1 in token
-// order.  The group's source rows do not depend on the slots, so every
-// thread issues the loads of its (at most kTileLoads) chunks of the tile
-// first; each wave then loads the bs slots itself (one per lane) and tests
-// them with a ballot, so the slot latency overlaps the data loads and no
-// barrier is needed to share the test.  Every wave reaches the same answer
-// from the same slots.
-// Row-major split (row-major tensors, whose groups write their own
-// tokens): the group's first k tokens end one block in order and the rest
-// start another, as in a prefill chunk that starts inside a block; the
-// loaded rows go straight to both blocks.
-// Shifted (other layouts, block sizes up to 32, where owned_runs decides
-// ownership): a prefill chunk that starts inside a block makes the group's
-// first k tokens continue the run of token t0 - 1 and its next bs tokens
-// fill the following block; the group then owns exactly that block (one
-// run starting at t0 + k).  k follows from the first test's slot of t0, so the
-// loads of rows t0 + k .. are issued together with the slots that confirm
-// it, instead of after the run analysis and a barrier.
-// Returns false, having stored nothing, when the group is neither (or is
-// the short last group, or its tile needs more than one pass): the caller
-// then runs the general run analysis.  The speculative loads stay within the
-// io rows of tokens < num_tokens.
-template <class Op, bool IDX, bool ODD>
-__device__ __forceinline__ bool write_tile_block(const WriteArgs &a, const WriteTileArgs &wt,
-                                                 int64_t t0, int32_t tile, bool v,
-                                                 float uniform, char *lds) {
-  constexpr int kDstLog2 = Op::kDst == 16 ? 4 : Op::kDst == 8 ? 3 : Op::kDst == 4 ? 2
-                           : Op::kDst == 2 ? 1 : 0;
-  const int32_t bs = 1 << wt.bs_log2;
-  const int32_t region = wt.tw << wt.bs_log2;  // cache bytes of the tile
-  const int32_t total = region >> kDstLog2;    // chunks of the tile
-  if (t0 + bs > a.num_tokens || total > kTileLoads * (int32_t)blockDim.x) return false;
-  const int32_t run_log2 = v ? wt.run_log2[1] : wt.run_log2[0];
-  const char *io = v ? a.src_v : a.src_k;
-  const int tid = (int)threadIdx.x;
-  const int lane = tid & (kWave - 1);
-  int64_t slot = -1;
-  if (lane < bs) slot = load_index(a.slots, t0 + lane, a.slot_is64);
-
-  // Source of chunk u for a run starting at token tb.  Row-major cache: the
-  // tile is bytes [tile * region, (tile + 1) * region) of the block, which
-  // hold io elements e = byte >> cache_es_log2 counted from row tb.
-  // Otherwise: chunk u is chunk tile_col(u) of the tile's columns of row
-  // tb + tile_row(u).
-  const int32_t cpr_log2 = wt.tw_log2 - kDstLog2;
-  const uint32_t e0 = ((uint32_t)tile * (uint32_t)wt.tw) >> wt.cache_es_log2;
-  auto row_of = [&](int32_t u) { return tile_row<ODD>(u, cpr_log2, wt); };
-  auto col_of = [&](int32_t u) { return tile_col<ODD>(u, row_of(u), cpr_log2, wt); };
-  auto elem = [&](int32_t u) -> uint32_t {  // io element of chunk u within its row run
-    return run_log2 < 0
-               ? (uint32_t)((tile * region + (u << kDstLog2)) >> wt.cache_es_log2)
-               : e0 + ((uint32_t)(col_of(u) << kDstLog2) >> wt.cache_es_log2);
+  // LDS: rows, then each row's offset and (narrow) the unit and token lists
+  const int32_t lrows = t.rows + (lane0 ? t.align : 0);
+  int64_t *s_off = reinterpret_cast<int64_t *>(lds + lrows * t.pitch);
+  auto stage = [&](const Raw<Op::kSrc> &v, int32_t u, int32_t r, bool in) {
+    const float sc = scale_of_chunk(u, r, in);
+    if (in) st<Op::kDst>(lds + r * t.pitch + (u - r * t.cpr) * Op::kDst, Op::apply(v, sc));
   };
-  Raw<Op::kSrc> x[kTileLoads];
-  auto load_rows = [&](int64_t tb) {
-    const char *src = io + tb * a.row_bytes;
-#pragma unroll
-    for (int k = 0; k < kTileLoads; ++k) {
-      const int32_t u = tid + k * (int32_t)blockDim.x;
-      if (u < total) {
-        x[k] = ld<Op::kSrc, kWriteNtLoad>(
-            run_log2 < 0 ? src + ((int64_t)elem(u) << wt.io_es_log2)
-                         : src + (int64_t)row_of(u) * a.row_bytes +
-                               ((int64_t)elem(u) << wt.io_es_log2));
-      }
-    }
-  };
-  auto uniform64 = [](int64_t x) {
-    return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) |
-                     (uint32_t)__builtin_amdgcn_readfirstlane((int)x));
-  };
-  load_rows(t0);
+  const uint32_t r0 = t.run_log2 >= 0 ? (uint32_t)c0 >> t.run_log2 : (uint32_t)c0 / (uint32_t)t.run;
+  char *dst = t.dst + (int64_t)r0 * t.s_run;
 
-  const int64_t first = uniform64(slot);
-  int64_t block = first >> wt.bs_log2;
-  const bool in_order = lane >= bs || slot == first + lane;
-  if (run_log2 < 0 && (__ballot(!in_order) != 0 || (first & (bs - 1)) != 0)) {
-    // Row-major split: tokens t0 .. t0 + k - 1 end block A (offsets
-    // bs - k .. bs - 1) and t0 + k .. t0 + bs - 1 start block B; the rows
-    // loaded above are this group's own, stored straight to both blocks.
-    if (first < 0 || block >= a.num_blocks || (first & (bs - 1)) == 0) return false;
-    const int32_t k = bs - (int32_t)(first & (bs - 1));
-    const int64_t f2 = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(
-                                      __shfl((int)(slot >> 32), k)) << 32) |
-                                 (uint32_t)__builtin_amdgcn_readfirstlane(__shfl((int)slot, k)));
-    const int64_t block_b = f2 >> wt.bs_log2;
-    const bool bad = lane < k ? slot != first + lane : (lane < bs && slot != f2 + (lane - k));
-    if (__ballot(bad) != 0 || f2 < 0 || (f2 & (bs - 1)) != 0 || block_b >= a.num_blocks)
-      return false;
-    const ScaleRef &sr = v ? a.vsc : a.ksc;
-    const uint32_t hd = (uint32_t)a.head_dim;
-    const uint32_t re = (uint32_t)a.nchunks * (uint32_t)a.chunk_elems;  // H * D
-    const int32_t rbc = wt.tiles * wt.tw;  // cache bytes of a row
-    char *base = v ? a.dst_v : a.dst_k;
-    const int64_t sb = v ? a.gv.s_block : a.gk.s_block;
-    // byte m of the group's rows: row m / rbc of the group is row
-    // bs - k + m / rbc of block A, or row m / rbc - k of block B
-    const int64_t at_a = block * sb + (int64_t)(bs - k) * rbc;
-    const int64_t at_b = block_b * sb - (int64_t)k * rbc;
-#pragma unroll
-    for (int q = 0; q < kTileLoads; ++q) {
-      const int32_t u = tid + q * (int32_t)blockDim.x;
-      if (u < total) {
-        const int32_t m = tile * region + (u << kDstLog2);
-        const bool in_a = m < k * rbc;
-        float sc = uniform;
-        if constexpr (Op::kScaled && IDX)
-          sc = scale_in_rows(sr, uniform, in_a ? block : block_b, elem(u), re, hd);
-        st<Op::kDst, kWriteNtStore>(base + ((in_a ? at_a : at_b) + m), Op::apply(x[q], sc));
-      }
+  // bit l of next: lane l's token follows lane l - 1's in its block
+  const int64_t prev = shfl64(slot, lane == 0 ? 0 : lane - 1);
+  const uint64_t oks = __ballot(ok);
+  const uint64_t next = __ballot(ok && lane > 0 && ((oks >> ((lane - 1) & 63)) & 1ull) != 0 &&
+                                 slot == prev + 1 && o != 0);
+  // The lanes whose tokens this workgroup stores: [first, end).
+  int32_t first = 0;
+  int32_t end = left;
+  if (lane0) {
+    // starts: lanes that go on with no aligned unit of `align` slots
+    const uint64_t starts = ~(next & __ballot((o & (t.align - 1)) != 0));
+    const uint64_t group = (starts >> 1) & ((1ull << t.rows) - 1ull);  // bit r: row r
+    if (group == 0) return;  // every row goes on with an earlier workgroup's
+    first = __ffsll((long long)group);  // the lane of that row
+    end = lane0 + left;
+    if (left == t.rows) {
+      const uint64_t after = starts & ~((1ull << (t.rows + 1)) - 1ull);
+      end = after ? __ffsll((long long)after) - 1 : kWave;
     }
-    return true;
   }
-  if (__ballot(!in_order) != 0 || first < 0 || (first & (bs - 1)) != 0 ||
-      block >= a.num_blocks) {
-    // Shifted: tokens t0 .. t0 + k - 1 hold first, first + 1, ... up to the
-    // end of its block and continue token t0 - 1 (first - 1); tokens t0 + k
-    // .. t0 + k + bs - 1 fill one block in order.
-    if (wt.bs_log2 > 5 || t0 == 0 || first < 0 || block >= a.num_blocks) return false;
-    const int32_t k = bs - (int32_t)(first & (bs - 1));
-    if (k >= bs || t0 + k + bs > a.num_tokens) return false;
-    if (__ballot(lane < k && slot != first + lane) != 0) return false;
-    const int64_t prev = load_index(a.slots, t0 - 1, a.slot_is64);
-    int64_t next = -1;
-    if (lane < bs) next = load_index(a.slots, t0 + k + lane, a.slot_is64);
-    load_rows(t0 + k);
-    const int64_t f2 = uniform64(next);
-    block = f2 >> wt.bs_log2;
-    if (prev != first - 1 || __ballot(lane < bs && next != f2 + lane) != 0 || f2 < 0 ||
-        (f2 & (bs - 1)) != 0 || block >= a.num_blocks)
-      return false;
-  }
-
-  const ScaleRef &sr = v ? a.vsc : a.ksc;
-  const uint32_t hd = (uint32_t)a.head_dim;
-  char *blk = v ? a.dst_v + block * a.gv.s_block : a.dst_k + block * a.gk.s_block;
-  if (run_log2 < 0) {
-    const uint32_t re = (uint32_t)a.nchunks * (uint32_t)a.chunk_elems;  // H * D
+  // rows past the workgroup's own tokens
+  const int32_t more = end - lane0 > t.rows ? end - lane0 - t.rows : 0;
+  Raw<Op::kSrc> y[kTileLoads];
 #pragma unroll
-    for (int k = 0; k < kTileLoads; ++k) {
-      const int32_t u = tid + k * (int32_t)blockDim.x;
-      if (u < total) {
-        float sc = uniform;
-        if constexpr (Op::kScaled && IDX) sc = scale_in_rows(sr, uniform, block, elem(u), re, hd);
-        st<Op::kDst, kWriteNtStore>(blk + tile * region + (u << kDstLog2), Op::apply(x[k], sc));
-      }
+  for (int k = 0; k < kTileLoads; ++k) {
+    const int32_t u = tid + k * nt;
+    if (u < more * t.cpr) {
+      const int32_t r = (int32_t)div_or_same((uint32_t)u, t.cpr_magic);
+      y[k] = ld<Op::kSrc, kWriteNtLoad>(src + (t.rows + r) * a.row_bytes +
+                                        (int64_t)(u - r * t.cpr) * Op::kSrc);
     }
-    return true;
   }
 #pragma unroll
   for (int k = 0; k < kTileLoads; ++k) {
-    const int32_t u = tid + k * (int32_t)blockDim.x;
-    if (u < total) {
-      float sc = uniform;
-      if constexpr (Op::kScaled && IDX) sc = scale_at(sr, uniform, block, elem(u), hd);
-      st<Op::kDst>(lds + row_of(u) * wt.pitch + (col_of(u) << kDstLog2), Op::apply(x[k], sc));
-    }
+    if (k * nt >= total) break;
+    stage(x[k], tid + k * nt, row[k], tid + k * nt < total);
   }
-  __syncthreads();
-  GroupRun r;
-  r.block = block;
-  r.lo = 0;
-  r.hi = bs;
-  r.tok = 0;
-  r.pad_ = 0;
-  unstage_any<true, ODD>(blk + (int64_t)tile * region, lds, region, run_log2, wt, r, v);
-  return true;
-}
+#pragma unroll
+  for (int k = 0; k < kTileLoads; ++k) {
+    if (k * nt >= more * t.cpr) break;
+    const int32_t u = tid + k * nt;
+    const int32_t r = t.rows + (int32_t)div_or_same((uint32_t)u, t.cpr_magic);
+    stage(y[k], t.rows * t.cpr + u, r, u < more * t.cpr);
+  }
+  if (tid < kWave && lane >= lane0 && lane - lane0 < lrows) s_off[lane - lane0] = off;
 
-// Op: the tile's chunk op (16-byte cache chunks); TokOp: the per-token
-// path's op, whose chunk fits the cache geometry (WriteArgs' chunking).
-// IDX: indexed (per-head / per-block) scales are looked up per chunk; the
-// per-tensor instances carry no lookup code (registers decide occupancy).
-template <class Op, class TokOp, bool IDX, bool ODD>
-__global__ __launch_bounds__(kBlockThreads) void write_tiles_kernel(WriteArgs a,
-                                                                    WriteTileArgs wt) {
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  __shared__ GroupRun s_runs[kMaxRuns];
-  __shared__ int32_t s_nruns;
-  const uint32_t gu = blockIdx.x / (uint32_t)wt.tiles;
-  const int32_t tile = (int32_t)(blockIdx.x - gu * (uint32_t)wt.tiles);
-  const int64_t t0 = (int64_t)gu << wt.bs_log2;
-  const bool v = blockIdx.y != 0;
-  float ks = 1.0f;  // per-tensor values; indexed scales are looked up per chunk
-  float vs = 1.0f;
-  if constexpr (Op::kScaled) {
-    ks = a.ksc.p[0];
-    vs = a.vsc.p[0];
-  }
-  if (write_tile_block<Op, IDX, ODD>(a, wt, t0, tile, v, v ? vs : ks, lds)) return;
-  // Which tokens this tensor's workgroups of the group write.  Row-major
-  // blocks (NHD) hold whole rows: each group writes its own tokens, split
-  // into runs (group_runs), so a block that a prefill chunk starts inside is
-  // written in two parts of whole rows.  Other layouts interleave a block's
-  // rows in 1-16 byte pieces; there, for block sizes up to 32, the group in
-  // which a run starts writes all of it (owned_runs), so that no cache line
-  // of a block is written in parts by two workgroups.
-  __shared__ int32_t s_own[2];
-  const int32_t run_log2 = v ? wt.run_log2[1] : wt.run_log2[0];
-  if (wt.bs_log2 <= 5 && run_log2 >= 0) {
-    owned_runs(a, t0, wt.bs_log2, s_runs, &s_nruns, s_own);
-  } else {
-    group_runs(a, t0, wt.bs_log2, s_runs, &s_nruns);
-    if (threadIdx.x == 0) {
-      s_own[0] = 0;
-      s_own[1] = 1 << wt.bs_log2;
-    }
-  }
-  __syncthreads();
-  const int32_t nruns = s_nruns;
-  if (nruns == 0) {
-    const int wpb = (int)(blockDim.x / kWave);  // waves per workgroup
-    write_group_tokens<TokOp, IDX>(a, t0 + s_own[0], s_own[1] - s_own[0], v, v ? vs : ks,
-                                   tile * wpb, wt.tiles * wpb);
+  if (!NARROW || t.kind == kTileStaged) {
+    __syncthreads();
+    // Piece u: the token fastest over the lanes, for runs of 16 bytes; longer
+    // runs keep their own 16-byte pieces together.
+    const int32_t pieces = t.run >> 4;  // of a run
+    const int32_t lo = first - lane0;
+    const int32_t hi = end - lane0;
+    auto store = [&](int32_t r1, int32_t n_log2) {  // rows [r1, r1 + 2^n_log2) below hi
+      const int32_t n = (t.tw >> 4) << n_log2;
+      for (int32_t u = tid; u < n; u += nt) {
+        const int32_t q = t.run_log2 >= 0 ? u >> (t.run_log2 - 4) : u / pieces;
+        const int32_t p = u - q * pieces;
+        const int32_t r = r1 + (q & ((1 << n_log2) - 1));
+        const int32_t j = q >> n_log2;
+        if (r >= hi) continue;
+        const int64_t ro = s_off[r];
+        if (ro >= 0)
+          st<16, kWriteNtStore>(dst + ro + (int64_t)j * t.s_run + p * 16,
+                                ld<16>(lds + r * t.pitch + j * t.run + p * 16));
+      }
+    };
+    store(lo, t.rows_log2);
+    // a run of rows that starts late in the tile and outlasts it
+    if (hi - lo > t.rows) store(lo + t.rows, 31 - __clz(t.align));
     return;
   }
-  for (int32_t i = 0; i < nruns; ++i) {
-    if (i > 0) __syncthreads();  // the LDS tile is reused
-    write_tile_run<Op, IDX, ODD>(a, wt, s_runs[i], t0, tile, v, v ? vs : ks, lds);
+
+  if constexpr (NARROW) {
+    int32_t *s_tab = reinterpret_cast<int32_t *>(s_off + lrows);
+    const uint64_t own = (end >= kWave ? ~0ull : (1ull << end) - 1ull) & (~0ull << first);
+    const uint64_t want = (1ull << (t.seg - 1)) - 1ull;
+    const bool head = ok && t.seg > 1 && (o & (t.seg - 1)) == 0 && lane < kWave - 1 &&
+                      lane + t.seg <= kWave && ((next >> ((lane + 1) & 63)) & want) == want;
+    const uint64_t heads = __ballot(head) & own;
+    uint64_t covered = heads;
+    for (int s = 1; s < t.seg; s *= 2) covered |= covered << s;
+    const uint64_t rest = oks & own & ~covered;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const int32_t units = __popcll(heads);
+    if (tid < kWave) {
+      const int32_t r = lane - lane0;
+      if ((heads >> lane) & 1ull) s_tab[__popcll(heads & below)] = r;
+      if ((rest >> lane) & 1ull) s_tab[units + __popcll(rest & below)] = r;
+    }
+    __syncthreads();
+    const int32_t *tokens = s_tab + units;
+    const int32_t ntok = __popcll(rest);
+    switch (t.run) {
+      case 1:
+        if (t.seg == 16) store_units<1, 16>(t, lds, s_off, s_tab, units, dst);
+        else if (t.seg == 8) store_units<1, 8>(t, lds, s_off, s_tab, units, dst);
+        store_tokens<1>(t, lds, s_off, tokens, ntok, dst);
+        break;
+      case 2:
+        if (t.seg == 8) store_units<2, 8>(t, lds, s_off, s_tab, units, dst);
+        store_tokens<2>(t, lds, s_off, tokens, ntok, dst);
+        break;
+      case 4:
+        if (t.seg == 4) store_units<4, 4>(t, lds, s_off, s_tab, units, dst);
+        store_tokens<4>(t, lds, s_off, tokens, ntok, dst);
+        break;
+      default:
+        if (t.seg == 2) store_units<8, 2>(t, lds, s_off, s_tab, units, dst);
+        store_tokens<8>(t, lds, s_off, tokens, ntok, dst);
+        break;
+    }
   }
 }
 
@@ -2477,20 +2170,19 @@ __global__ __launch_bounds__(kFlatThreads) void gather_ragged_tile_kernel(Gather
 // ---------------------------------------------------------------------------
 // Launch templates.
 
-// How a write launches: the per-token kernel, or the tiled block kernel
-// (one workgroup per tile of a group's block, per tensor) with its LDS
-// tile size.
+// How a write launches: the per-token kernel, the flat kernel, or the tile
+// kernel with its LDS size.
 struct WriteLaunch {
   int grid;
   int64_t flat_grid;  // write_flat_kernel's workgroups, 0 when it does not apply
   bool tiles;
   WriteTileArgs wt;
   int64_t tile_grid;
+  int32_t tile_threads;
   uint32_t tile_lds;
 };
 
-// The tiled write moves 16-byte cache chunks: a copy of 16 bytes, or a
-// quantization of 8 elements.
+// The tiled write moves 16-byte cache chunks, or quantizes 8 elements.
 template <class Op>
 struct TileOpOf;
 template <int B>
@@ -2502,29 +2194,26 @@ struct TileOpOf<QuantOp<G, IO, F8>> {
   using type = QuantOp<8, IO, F8>;
 };
 
+template <class TOp, bool IDX>
+void launch_write_tiles(const WriteLaunch &w, hipStream_t s) {
+  const dim3 g((uint32_t)w.tile_grid, 2), b(w.tile_threads);
+  if (w.wt.t[0].kind == kTileNarrow || w.wt.t[1].kind == kTileNarrow)
+    hipLaunchKernelGGL((write_tiles_kernel<TOp, IDX, true>), g, b, w.tile_lds, s, w.wt);
+  else
+    hipLaunchKernelGGL((write_tiles_kernel<TOp, IDX, false>), g, b, w.tile_lds, s, w.wt);
+}
+
 template <class Op>
 void launch_write_op(const WriteArgs &a, const WriteLaunch &w, hipStream_t s) {
   if (w.tiles) {
     using TOp = typename TileOpOf<Op>::type;
-    const dim3 g((uint32_t)w.tile_grid, 2);
-    const bool odd = w.wt.tw_log2 < 0;  // tile width not a power of two
     if constexpr (Op::kScaled) {
       if (a.ksc.indexed || a.vsc.indexed) {
-        if (odd)
-          hipLaunchKernelGGL((write_tiles_kernel<TOp, Op, true, true>), g, dim3(w.wt.threads),
-                             w.tile_lds, s, a, w.wt);
-        else
-          hipLaunchKernelGGL((write_tiles_kernel<TOp, Op, true, false>), g, dim3(w.wt.threads),
-                             w.tile_lds, s, a, w.wt);
+        launch_write_tiles<TOp, true>(w, s);
         return;
       }
     }
-    if (odd)
-      hipLaunchKernelGGL((write_tiles_kernel<TOp, Op, false, true>), g, dim3(w.wt.threads),
-                         w.tile_lds, s, a, w.wt);
-    else
-      hipLaunchKernelGGL((write_tiles_kernel<TOp, Op, false, false>), g, dim3(w.wt.threads),
-                         w.tile_lds, s, a, w.wt);
+    launch_write_tiles<TOp, false>(w, s);
   } else if (w.flat_grid > 0) {
     const dim3 g((uint32_t)w.flat_grid), b(kFlatThreads);
     if (a.nchunks_log2 >= 6) {
