@@ -19,6 +19,7 @@
 // downstream may depend on them.
 #pragma once
 
+#include <math.h>
 #include <stdint.h>
 #include <string.h>
 
@@ -156,6 +157,54 @@ KVX_HD float canon_nan_f32(float f) {
   return ((f32_bits(f) & 0x7FFFFFFFu) > 0x7F800000u) ? bits_f32(0x7FC00000u)
                                                     : f;
 }
+
+// x / s for the FP8 quantization, as two operations per element: 1 / s is
+// held as hi + lo, hi its truncation toward zero and lo the rest, and
+// quant_quotient returns fma(x, hi, x * lo).
+//
+// The FP8 code of that value equals the code of the correctly rounded f32
+// quotient.  hi + lo carries 1 / s to a relative 2^-45 and x * lo rounds at
+// 2^-47, so the exact value that the fma rounds is (x / s)(1 + d), |d| <
+// 2^-44.8.  It rounds to another float than x / s does only if a midpoint b
+// of two adjacent floats lies between them, and the codes of those two
+// floats differ only if one of them is a boundary m between FP8 codes (at
+// most 5 significant bits): b = m +- half an ulp.  With 24-bit significands
+// X of x and S of s and m = M / 16, |x / s - b| <= |d| x / s then says
+// |2^20 K -+ S| < 19 for an integer K, that is, S lies within 18 of a
+// multiple of 2^20.  Such scales (other than the multiples themselves, for
+// which the difference would have to be 0, which a 25-bit b times S cannot
+// give: x has 24 bits), and those outside [2^-60, 2^60], take the division
+// (fast = false).  lo carries hi's sign and is at least 2^-126, so signed
+// zeros and infinities of x come out as from the division; tiny quotients
+// that underflow are far below half the smallest code, and huge ones
+// saturate.
+struct QuantScale {
+  float s;
+  float hi;
+  float lo;
+  bool fast;
+};
+
+KVX_HD QuantScale quant_scale(float s) {
+  QuantScale q;
+  const uint32_t u = f32_bits(s);
+  const uint32_t a = u & 0x7FFFFFFFu;
+  const uint32_t low = u & 0xFFFFFu;  // S mod 2^20
+  q.s = s;
+  q.fast = a >= 0x21800000u && a <= 0x5D800000u && (low == 0 || low - 64u <= 0xFFFFFu - 127u);
+  float r = 1.0f / s;
+  float e = fmaf(-r, s, 1.0f);
+  if (e < 0.0f) {  // |r| > |1 / s|: one float toward zero
+    r = bits_f32(f32_bits(r) - 1u);
+    e = fmaf(-r, s, 1.0f);
+  }
+  const uint32_t l = f32_bits(e * r) & 0x7FFFFFFFu;
+  q.hi = r;
+  q.lo = bits_f32((u & 0x80000000u) | (l < 0x00800000u ? 0x00800000u : l));
+  return q;
+}
+
+KVX_HD float quant_quotient(const QuantScale &q, float x) { return fmaf(x, q.hi, x * q.lo); }
 
 KVX_HD float f16_to_f32(uint16_t h) {
   const uint32_t sign = (uint32_t)(h & 0x8000u) << 16;

@@ -284,23 +284,47 @@ __device__ __forceinline__ float io_to_f32(const Raw<B> &x, int i) {
   } else if constexpr (IO == KVX_DTYPE_BF16) {
     return bf16_to_f32((uint16_t)get16(x, i));
   } else {
-    return f16_to_f32((uint16_t)get16(x, i));
-  }
-}
-
-template <int IO, int B>
-__device__ __forceinline__ void f32_to_io(float v, Raw<B> &y, int i) {
-  if constexpr (IO == KVX_DTYPE_F32) {
-    y.w[i] = f32_bits(canon_nan_f32(v));
-  } else if constexpr (IO == KVX_DTYPE_BF16) {
-    put16(y, i, f32_to_bf16(v));
-  } else {
-    put16(y, i, f32_to_f16(v));
+    // exact for every finite value; NaN stays NaN (callers canonicalize)
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)get16(x, i));
   }
 }
 
 // io (F16/BF16/F32) -> FP8 (F8 = KVX_DTYPE_F8_E4M3 or KVX_DTYPE_F8_E5M2):
-// q = fp8(sat(x / scale)).
+// q = fp8(sat(x / scale)), byte for byte what fp_convert.h's f32_to_e4m3 /
+// f32_to_e5m2 give of the correctly rounded quotient.  The quotient is two
+// operations per element (quant_quotient; scales it does not cover divide),
+// gfx950's v_maximum3 / v_minimum3 clamp to the largest code and keep NaN,
+// v_cvt_pk_fp8_f32 / v_cvt_pk_bf8_f32 round two elements to nearest even,
+// and NaN codes, the only ones above the clamp's, become canonical.
+// Dividing and rounding in integer code took about 45 instructions per
+// element and bounded the quantizing writes.  On MI355X (rocprofv3, 19200
+// tokens of 8 x 128 bf16 into E4M3, us per launch, before -> after): NHD
+// 30.6 -> 22.3 (5.3 TB/s), 200 decode tokens 5.1 -> 3.3; in the tiled write
+// (76800 tokens, 16-token blocks) HND 110 -> 89, x-packed 119 -> 89.
+// BRANCH: a word without NaN, nearly every one, skips the correction.
+template <int F8, bool BRANCH>
+__device__ __forceinline__ uint32_t encode4(float q0, float q1, float q2, float q3) {
+  constexpr float kTop = F8 == KVX_DTYPE_F8_E5M2 ? 57344.0f : 448.0f;
+  auto clamp = [](float q) {
+    return __builtin_elementwise_minimum(__builtin_elementwise_maximum(q, -kTop), kTop);
+  };
+  int w = 0;
+  if constexpr (F8 == KVX_DTYPE_F8_E5M2) {
+    w = __builtin_amdgcn_cvt_pk_bf8_f32(clamp(q0), clamp(q1), w, false);
+    w = __builtin_amdgcn_cvt_pk_bf8_f32(clamp(q2), clamp(q3), w, true);
+  } else {
+    w = __builtin_amdgcn_cvt_pk_fp8_f32(clamp(q0), clamp(q1), w, false);
+    w = __builtin_amdgcn_cvt_pk_fp8_f32(clamp(q2), clamp(q3), w, true);
+  }
+  // bytes whose magnitude lies above the largest finite code (0x7E, 0x7B)
+  constexpr uint32_t kAbove = F8 == KVX_DTYPE_F8_E5M2 ? 0x04040404u : 0x01010101u;
+  constexpr uint32_t kNan = F8 == KVX_DTYPE_F8_E5M2 ? 0x7E7E7E7Eu : 0x7F7F7F7Fu;
+  const uint32_t nan = (((uint32_t)w & 0x7F7F7F7Fu) + kAbove) & 0x80808080u;
+  if (BRANCH && nan == 0) return (uint32_t)w;
+  const uint32_t m = (nan << 1) - (nan >> 7);  // 0xFF in each such byte
+  return ((uint32_t)w & ~m) | (kNan & m);
+}
+
 template <int G, int IO, int F8>
 struct QuantOp {
   static constexpr int kSrc = G * IoType<IO>::kBytes;
@@ -308,14 +332,21 @@ struct QuantOp {
   static constexpr bool kScaled = true;
   __device__ __forceinline__ static Raw<kDst> apply(const Raw<kSrc> &x,
                                                     float scale) {
+    const QuantScale qs = quant_scale(scale);
+    float q[G < 4 ? 4 : G];
+#pragma unroll
+    for (int i = G; i < 4; ++i) q[i] = 0.0f;
+    if (qs.fast) {
+#pragma unroll
+      for (int i = 0; i < G; ++i) q[i] = quant_quotient(qs, io_to_f32<IO>(x, i));
+    } else {
+#pragma unroll
+      for (int i = 0; i < G; ++i) q[i] = io_to_f32<IO>(x, i) / scale;
+    }
     Raw<kDst> y;
 #pragma unroll
-    for (int k = 0; k < Raw<kDst>::kWords; ++k) y.w[k] = 0;
-#pragma unroll
-    for (int i = 0; i < G; ++i) {
-      const float q = io_to_f32<IO>(x, i) / scale;
-      put8(y, i, F8 == KVX_DTYPE_F8_E5M2 ? f32_to_e5m2(q) : f32_to_e4m3(q));
-    }
+    for (int k = 0; k < Raw<kDst>::kWords; ++k)
+      y.w[k] = encode4<F8, (G >= 4)>(q[4 * k], q[4 * k + 1], q[4 * k + 2], q[4 * k + 3]);
     return y;
   }
 };
