@@ -345,6 +345,19 @@ constexpr int64_t kWriteAlignBytes = 64;
 // inside blocks and on them), 512 bytes 117 and 117.
 constexpr int64_t kWriteDirectWidth = 2048;
 
+// Row-major pairs take this kernel (both tensors direct: four chunks of one
+// tensor per lane where write_flat_kernel has one of each) when the bytes
+// they read and write lie within these bounds, about what the 256 MB
+// Infinity Cache holds of them.  NHD, flat -> tiles: 8 x 128 bf16, 1000 /
+// 4000 / 10000 / 30000 tokens 3.19 / 8.28 / 16.97 / 47.25 -> 3.56 / 7.09 /
+// 13.93 / 46.43; into E4M3 4000 / 10000 / 30000 tokens 7.50 / 14.52 / 34.65
+// -> 7.64 / 12.46 / 34.69; 1 x 576 bf16, 30000 tokens 26.6 -> 24.3; 8 x 256
+// f32, 4000 / 10000 tokens 24.4 / 58.4 -> 21.2 / 60.9.
+constexpr int64_t kWriteRowsMin = 12 << 20;
+constexpr int64_t kWriteRowsMax = 256 << 20;
+constexpr int64_t kWriteRowsMinQuant = 32 << 20;
+constexpr int64_t kWriteRowsMaxQuant = 192 << 20;
+
 // The divisor of `row` that is a multiple of `unit` and at most `target`,
 // the widest of whole 128-byte lines first; the narrowest one when all are
 // wider than target.
@@ -386,8 +399,12 @@ bool plan_write_tiles(const WritePlan &p, int cs, int is, WriteTileArgs *wt, int
     run_elems[i] = dense_run_elems(*g[i], bs, H, D);
     if (run_elems[i] < 0) return false;
   }
-  // row-major pairs: the flat kernel
-  if (run_elems[0] == H * D && run_elems[1] == H * D) return false;
+  if (run_elems[0] == H * D && run_elems[1] == H * D) {
+    const int64_t bytes = 2 * p.num_tokens * (row + H * D * is);
+    if (bytes < (quant ? kWriteRowsMinQuant : kWriteRowsMin) ||
+        bytes > (quant ? kWriteRowsMaxQuant : kWriteRowsMax))
+      return false;  // the flat kernel
+  }
   int64_t base_tile = kWriteTileBytes;
   while (base_tile > kWriteTileMin && p.num_tokens * row / base_tile < kWriteTileWorkgroups)
     base_tile /= 2;

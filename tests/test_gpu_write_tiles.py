@@ -114,3 +114,19 @@ def test_one_chunk_from_every_phase(layout, start):
     slots = ids[pos // bs] * bs + pos % bs
     key, val = (torch.randn((T, H, D), generator=gen).bfloat16().to(DEV) for _ in range(2))
     check_write(pc, kb, vb, key, val, slots.to(DEV), io_dtype=DType.BF16, cache_dtype=DType.BF16)
+
+
+@pytest.mark.parametrize("fp8,tokens", [(None, 3200), (None, 1500), (DType.F8_E4M3, 5600),
+                                        (DType.F8_E4M3, 2800)])
+@pytest.mark.parametrize("bs", [16, 20])
+def test_row_major_pairs_by_size(fp8, tokens, bs):
+    """NHD pairs on both sides of the size rule that picks the kernel."""
+    rng = np.random.default_rng(tokens + bs)
+    gen = torch.Generator().manual_seed(tokens + bs)
+    H, D, nb = 8, 128, tokens // bs + 300
+    dtype = fp8 or DType.BF16
+    pc, kb, vb = make_cache(NHD, NHD, dtype, nb, bs, H, D, gen=gen)
+    s = slots_of("spoiled", tokens, bs, nb, rng)
+    key, val = (torch.randn((s.size, H, D), generator=gen).bfloat16().to(DEV) for _ in range(2))
+    check_write(pc, kb, vb, key, val, torch.from_numpy(s).to(DEV), io_dtype=DType.BF16,
+                cache_dtype=dtype, k_scale=0.01 if fp8 else None, v_scale=0.02 if fp8 else None)
