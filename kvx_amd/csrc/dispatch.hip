@@ -597,9 +597,11 @@ kvx_status_t enqueue_gather(const GatherPlan &p, void *stream) {
   };
   const bool ragged_tile =
       p.format == KVX_BLOCK_TABLE_RAGGED && rows_contig(p.gk) && rows_contig(p.gv);
+  // bytes of cache per chunk at most (FP8: kDequantChunk and its comment)
   const int max_bytes = p.conv != kConvDequant                               ? 16
-                        : p.format == KVX_BLOCK_TABLE_RAGGED && !ragged_tile ? kRaggedDequantChunk
-                                                                             : kDequantChunk;
+                        : p.format == KVX_BLOCK_TABLE_RAGGED && !ragged_tile && is != 4
+                            ? kRaggedDequantChunk
+                            : dequant_chunk(is);
   const void *base_k = p.src_k;
   const void *base_v = p.src_v;
   if (p.format == KVX_BLOCK_TABLE_KV_OFFSETS) {
@@ -629,7 +631,7 @@ kvx_status_t enqueue_gather(const GatherPlan &p, void *stream) {
     int64_t tgrid = 0;
     uint32_t tlds = 0;
     const bool dq = p.conv == kConvDequant;
-    if (p.seq_count > 0 && plan_tiles(p, cs, is, dq ? kDequantChunk : 16, &t, &tgrid, &tlds)) {
+    if (p.seq_count > 0 && plan_tiles(p, cs, is, dq ? dequant_chunk(is) : 16, &t, &tgrid, &tlds)) {
       if (tgrid == 0) return KVX_STATUS_OK;
       const bool i64 = p.lens_is64 != 0;
       const bool p64 = p.indptr_is64 != 0;

@@ -60,6 +60,9 @@ __device__ __forceinline__ uint32_t div_magic(uint32_t x, uint32_t m) { return _
 // the dequantizing gather (c4) 2% faster (256-thread, 4 KiB tiles).
 constexpr int kFlatUnroll = 1;
 constexpr int kFlatUnrollDequant = 2;
+// 4-code chunks (kDequantChunkF32; E4M3 to f32, 64000 tokens of 8 x 128, NHD
+// PACKED): 168, 122 and 119 us with one, two and four in flight.
+constexpr int kFlatUnrollDequantF32 = 4;
 // Non-temporal (streaming) cache loads and output stores in every gather:
 // together 4-13% faster than either alone.
 constexpr bool kGatherNtLoad = true;
@@ -116,6 +119,18 @@ constexpr int64_t kOffsetsTileCopyRow = 512;
 // every other gather, gather_ragged_tile_kernel included (8 bytes).
 constexpr int kDequantChunk = 8;
 constexpr int kRaggedDequantChunk = 16;
+// Into f32 they take four codes, so that a lane's chunk is one 16-byte store
+// and a wave's stores are whole lines: with eight, each of a chunk's two
+// 16-byte stores wrote half of every 32 bytes.  MI355X, E4M3 to f32, 64000
+// tokens of 8 x 128, us per gather, 8 -> 4 codes: NHD PACKED / RAGGED /
+// KV_OFFSETS 148 / 146 / 175 -> 119 / 119 / 124 (5.6 TB/s), HND 252 / 238 /
+// 250 -> 141 / 137 / 143, vLLM's pair PACKED 252 -> 142; HND 128-token blocks
+// RAGGED (16-code chunks before) 197 -> 159.
+constexpr int kDequantChunkF32 = 4;
+// Chunk of a dequantizing gather into io elements of io_size bytes.
+constexpr int dequant_chunk(int io_size) {
+  return io_size == 4 ? kDequantChunkF32 : kDequantChunk;
+}
 // Non-temporal io-row loads of the tiled block write (off) and of the
 // per-token write (on), and non-temporal cache stores of every write
 // kernel (on).  On MI355X (c3 shapes) non-temporal stores make the tiled
@@ -1153,13 +1168,20 @@ __device__ __forceinline__ const char *flat_src(const GatherArgs &a, const GeomB
   }
 }
 
+// Chunks per lane in flight.
+template <class Op>
+constexpr int flat_unroll() {
+  if (!Op::kScaled) return kFlatUnroll;
+  return Op::kSrc == kDequantChunkF32 ? kFlatUnrollDequantF32 : kFlatUnrollDequant;
+}
+
 // c0: chunk index of ck / cv counted from a row start (indexed scales).
 // HR: ck / cv are the blocks, the run's chunks addressed by flat_src.
 template <class Op, bool HR = false>
 __device__ __forceinline__ void flat_copy(const GatherArgs &a, const char *ck, const char *cv,
                                           char *ok, char *ov, int64_t total, float ks, float vs,
                                           int64_t bid, int64_t c0) {
-  constexpr int U = Op::kScaled ? kFlatUnrollDequant : kFlatUnroll;
+  constexpr int U = flat_unroll<Op>();
   const int64_t both = 2 * total;
   int64_t f = threadIdx.x;
   for (; f + (U - 1) * kFlatThreads < both; f += U * kFlatThreads) {
@@ -2110,7 +2132,7 @@ __global__ __launch_bounds__((indexed_flat_threads<Op, FMT>())) void gather_inde
 // end, and so does every later one.
 template <class Op, bool I64, bool P64>
 __device__ __forceinline__ bool ragged_tile_unit(const GatherArgs &a, int64_t s, int64_t t0) {
-  constexpr int U = Op::kScaled ? kFlatUnrollDequant : kFlatUnroll;
+  constexpr int U = flat_unroll<Op>();
   int64_t n;
   int64_t start;
   if (!indexed_extent<KVX_BLOCK_TABLE_RAGGED, I64, P64>(a, s, t0, n, start)) return false;
@@ -2354,8 +2376,8 @@ void launch_tiles_dequant(int io, const TileArgs &t, int fmt, bool i64, bool p64
                           uint32_t lds, hipStream_t s) {
   switch (io) {
     case KVX_DTYPE_F32:
-      launch_tiles<DequantOp<kDequantChunk, KVX_DTYPE_F32, F8>>(t, fmt, i64, p64, grid, lds,
-                                                                    s);
+      launch_tiles<DequantOp<kDequantChunkF32, KVX_DTYPE_F32, F8>>(t, fmt, i64, p64, grid, lds,
+                                                                       s);
       break;
     case KVX_DTYPE_F16:
       launch_tiles<DequantOp<kDequantChunk, KVX_DTYPE_F16, F8>>(t, fmt, i64, p64, grid, lds,
@@ -2381,9 +2403,11 @@ void dispatch_quant(int ge, const WriteArgs &a, const WriteLaunch &w, hipStream_
 template <int IO, int F8>
 void dispatch_dequant(int ge, const GatherArgs &a, int64_t grid,
                       hipStream_t s) {
+  if constexpr (IO != KVX_DTYPE_F32) {  // at most kDequantChunkF32 codes there
+    if (ge == 16) return launch_gather_op<DequantOp<16, IO, F8>>(a, grid, s);
+    if (ge == 8) return launch_gather_op<DequantOp<8, IO, F8>>(a, grid, s);
+  }
   switch (ge) {
-    case 16: launch_gather_op<DequantOp<16, IO, F8>>(a, grid, s); break;
-    case 8: launch_gather_op<DequantOp<8, IO, F8>>(a, grid, s); break;
     case 4: launch_gather_op<DequantOp<4, IO, F8>>(a, grid, s); break;
     case 2: launch_gather_op<DequantOp<2, IO, F8>>(a, grid, s); break;
     default: launch_gather_op<DequantOp<1, IO, F8>>(a, grid, s); break;
