@@ -160,8 +160,36 @@ def build_torch_ops(verbose: bool = False) -> Path:
     return TORCH_OPS_LIB
 
 
+PAGED_HOST_SRC = CSRC / "paged_host.cpp"
+PAGED_HOST_LIB = PKG_DIR / "_paged_host.so"
+
+
+def build_paged_host(verbose: bool = False) -> Path:
+    """Compile paged.py's descriptor builder (csrc/paged_host.cpp), a CPython
+    module over the installed torch.  Host code only."""
+    import sysconfig
+
+    import torch
+
+    tdir = Path(torch.__file__).resolve().parent
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    cxx = shutil.which("g++") or "g++"
+    tmp = PAGED_HOST_LIB.with_suffix(".so.tmp")
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+          "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+          f"-I{INCLUDE}", f"-I{sysconfig.get_paths()['include']}", f"-I{tdir / 'include'}",
+          f"-I{tdir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+          f"-I{rocm / 'include'}", str(PAGED_HOST_SRC), "-o", str(tmp),
+          f"-L{tdir / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip",
+          "-ltorch_python", f"-L{rocm / 'lib'}", "-lamdhip64"], verbose)
+    os.replace(tmp, PAGED_HOST_LIB)
+    return PAGED_HOST_LIB
+
+
 if __name__ == "__main__":
     print(build(verbose="-v" in sys.argv))
     print(build_bench(verbose="-v" in sys.argv))
     print(build_probe(verbose="-v" in sys.argv))
     print(build_torch_ops(verbose="-v" in sys.argv))
+    print(build_paged_host(verbose="-v" in sys.argv))

@@ -1,8 +1,9 @@
 """Torch-facing host helpers over the KVX C ABI.
 
 These build kvx_abi.h descriptors from torch tensors (shape, element strides,
-data pointer, memory type) and call libkvx_amd.so through ctypes.  torch is
-only the source of device memory and streams here; every byte is moved by the
+data pointer, memory type) and call libkvx_amd.so; ``write_kv`` and
+``gather_kv`` have them built natively (csrc/paged_host.cpp).  torch is only
+the source of device memory and streams here; every byte is moved by the
 library's HIP kernels.  There is no fallback: if libkvx_amd.so is missing,
 ``abi.load()`` raises.
 
@@ -14,12 +15,40 @@ return the kvx_status_t as ``abi.Status``.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 from dataclasses import dataclass
+from pathlib import Path
 
 import torch
 
 from . import abi
 from .abi import DType, Layout, Memory, Status
+
+_HOST_PATH = Path(__file__).resolve().parent / "_paged_host.so"
+_HOST = None
+_STATUS = {int(s): s for s in Status}
+
+
+def _host():
+    """The native descriptor builder (csrc/paged_host.cpp)."""
+    global _HOST
+    if _HOST is None:
+        if not _HOST_PATH.exists():
+            raise RuntimeError(f"{_HOST_PATH} is missing; build it with `python -m kvx_amd.build`")
+        spec = importlib.util.spec_from_file_location("_paged_host", _HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _HOST = module
+    return _HOST
+
+
+def _address(lib, name: str) -> int:
+    """Address of an entry point of the loaded library."""
+    known = lib.__dict__.setdefault("_kvx_addresses", {})
+    if name not in known:
+        known[name] = C.cast(getattr(lib, name), C.c_void_p).value
+    return known[name]
+
 
 _TORCH_DTYPE = {
     torch.float16: DType.F16,
@@ -188,6 +217,18 @@ def scale_desc_of(scale) -> abi.ScaleDesc:
     return abi.scale_desc(scale.data_ptr())
 
 
+def _cache_args(cache: PagedCache) -> tuple:
+    return (cache.key_cache, cache.value_cache, cache.k_layout, cache.v_layout, cache.num_blocks,
+            cache.block_size, cache.heads, cache.head_dim)
+
+
+def _scale_args(scale) -> tuple:
+    """(tensor, granularity) of a scale; -1: a per-tensor tensor."""
+    if isinstance(scale, Scales):
+        return scale.values, int(scale.granularity)
+    return scale, -1
+
+
 def build_write(cache: PagedCache, key: torch.Tensor, value: torch.Tensor,
                 slot_mapping: torch.Tensor, k_scale=None, v_scale=None) -> abi.WriteDesc:
     """kvx_write_desc_t for [T, H, D] key/value rows and [T] slots.  FP8
@@ -323,6 +364,17 @@ def write_kv(cache: PagedCache, key: torch.Tensor, value: torch.Tensor,
     """Scatter rows into the paged cache.  entry = "launch" (kvx_paged_kv.h)
     or "abi" (kvx_write_kv of kvx_abi.h)."""
     lib = abi.load()
+    name = ("kvx_write_kv" if entry == "abi" else "kvx_launch_write_kv"
+            if tokens_per_seq is None else "kvx_launch_write_kv_prefill")
+    code = None
+    if type(cache) is PagedCache:
+        code = _host().write(
+            _address(lib, name), None if entry == "abi" else tokens_per_seq,
+            None if stream is None else _stream_handle(stream), *_cache_args(cache), key, value,
+            slot_mapping, *_scale_args(k_scale), *_scale_args(v_scale))
+    if code is not None:
+        return _STATUS[code]
+    # arguments that the native builder leaves to the descriptor helpers
     cd = cache.desc()
     wd = build_write(cache, key, value, slot_mapping, k_scale, v_scale)
     s = _stream_handle(stream)
@@ -346,6 +398,22 @@ def gather_kv(cache: PagedCache, key_out: torch.Tensor, value_out: torch.Tensor,
     (kvx_launch_gather_kv_dequant).  pool_blocks = (primary, secondary)
     block counts go through kvx_launch_gather_kv_pools instead."""
     lib = abi.load()
+    if type(cache) is PagedCache and pool_blocks is None and (entry != "abi" or k_scale is None):
+        if isinstance(block_table, RaggedTable):
+            table = (block_table.indices, block_table.indptr, None, None, 0)
+        elif isinstance(block_table, OffsetsTable):
+            table = (block_table.offsets, None, block_table.primary, block_table.secondary,
+                     block_table.bytes_per_block)
+        else:
+            table = (block_table, None, None, None, 0)
+        name = ("kvx_gather_kv" if entry == "abi" else "kvx_launch_gather_kv"
+                if k_scale is None and v_scale is None else "kvx_launch_gather_kv_dequant")
+        code = _host().gather(
+            _address(lib, name), None if stream is None else _stream_handle(stream),
+            *_cache_args(cache), key_out, value_out, *table, seq_lens, max_seq_len, *_scale_args(k_scale), *_scale_args(v_scale))
+        if code is not None:
+            return _STATUS[code]
+    # arguments that the native builder leaves to the descriptor helpers
     cd = gather_cache_desc(cache, block_table)
     gd = build_gather(key_out, value_out, block_table, seq_lens, max_seq_len)
     s = _stream_handle(stream)
