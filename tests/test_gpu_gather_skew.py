@@ -1,0 +1,52 @@
+"""GPU parity of gathers whose grid mostly lies past the sequences: every
+table format with lengths of 0, negative, cut inside a tile and past max_seq_len."""
+import numpy as np
+import pytest
+import torch
+
+from kvx_amd import paged
+from kvx_amd.abi import DType, Layout
+
+from gpu_helpers import (TORCH_DT, OffsetsPool, check_gather, check_gather_offsets,
+                         check_gather_ragged, make_cache, random_fill)
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+NHD, HND, PK = Layout.BLOCK_NHD, Layout.BLOCK_HND, Layout.BLOCK_HND_PACKED
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("table", ["packed", "ragged", "offsets"])
+@pytest.mark.parametrize("layout,bs", [(NHD, 16), (HND, 16), (HND, 64), (PK, 32), (NHD, 24)])
+def test_lengths_at_every_edge(layout, bs, table, fp8):
+    if table == "offsets" and bs == 24:
+        pytest.skip("KV_OFFSETS blocks are a power of two")
+    rng = np.random.default_rng(bs + fp8)
+    gen = torch.Generator().manual_seed(bs)
+    dtype, io = (DType.F8_E4M3, DType.BF16) if fp8 else (DType.BF16, DType.BF16)
+    H, D, L, nb = 8, 128, 700, 90
+    edges = [0, -1, 1, bs - 1, bs, bs + 1, 2 * bs, L - 1, L, L + 1, 8 * bs + 3]
+    S, mbps = len(edges), -(-L // bs)
+    lens = torch.tensor(edges, dtype=torch.int32, device=DEV)
+    ko = random_fill(torch.empty((S, L, H, D), dtype=TORCH_DT[io], device=DEV), gen)
+    vo = random_fill(torch.empty_like(ko), gen)
+    sc = dict(k_scale=0.02, v_scale=0.03) if fp8 else {}
+    kw = dict(cache_dtype=dtype, io_dtype=io, **sc)
+    ids = rng.integers(-1, nb + 1, size=(S, mbps)).astype(np.int32)
+    pack = 16 if fp8 else 8
+    if table == "offsets":
+        pool = OffsetsPool(layout, layout, dtype, nb, bs, H, D, pack=pack, gen=gen)
+        raw = rng.integers(0, nb + 2, size=(S, 1, 2, mbps)).astype(np.uint32)
+        raw |= (rng.random(raw.shape) < 0.3).astype(np.uint32) << 31
+        check_gather_offsets(pool, ko, vo, torch.from_numpy(raw.view(np.int32)).to(DEV), lens, L,
+                             **kw)
+        return
+    pc, kb, vb = make_cache(layout, layout, dtype, nb, bs, H, D, pack=pack, gen=gen)
+    if table == "packed":
+        check_gather(pc, kb, vb, ko, vo, torch.from_numpy(ids).to(DEV), lens, L, **kw)
+        return
+    rows = np.repeat(ids, bs, axis=1)[:, :L]
+    indptr = (np.arange(S + 1) * L).astype(np.int32)
+    check_gather_ragged(pc, kb, vb, ko, vo,
+                        paged.RaggedTable(torch.from_numpy(rows.reshape(-1).copy()).to(DEV),
+                                          torch.from_numpy(indptr).to(DEV)), lens, L, **kw)
