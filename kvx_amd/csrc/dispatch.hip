@@ -721,6 +721,12 @@ kvx_status_t enqueue_gather(const GatherPlan &p, void *stream) {
       int64_t want = kFlatTileBytes / (row_elems * cs);
       int64_t r = 1;
       while (r * 2 <= want && r * 2 <= kWave && p.block_size % (r * 2) == 0) r *= 2;
+      // a large batch whose table holds few of the rows the grid covers (one
+      // entry per token: skewed lengths): tiles of twice the rows
+      const int64_t entries = p.table_count;
+      if (entries * kRaggedSparse < (int64_t)p.seq_count * p.max_seq_len &&
+          entries >= r * kRaggedSparseTiles && r * 2 <= kWave && p.block_size % (r * 2) == 0)
+        r *= 2;
       a.ragged_tile = 1;
       a.rows_per_wg = (int32_t)r;
       a.blocks_per_seq = (int32_t)(((int64_t)p.max_seq_len + r - 1) / r);

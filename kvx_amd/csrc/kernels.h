@@ -1274,6 +1274,16 @@ constexpr uint32_t kFlatLongLds = 12800;
 // of at least kFlatHeadRunsMinBs tokens take gather_flat_kernel with
 // head-run addressing instead of the LDS tiles or the row kernel.
 constexpr int kFlatHeadRunsMinBs = 64;
+// Tiles of twice the rows, half the workgroups, when a RAGGED table has fewer
+// entries than 1 / kRaggedSparse of the rows the grid covers and fills at
+// least kRaggedSparseTiles tiles: most workgroups then find no rows.  On
+// MI355X (log-uniform lengths, us per gather): MLA rows, 96 sequences up to
+// 16384 tokens, 344 -> 293; 128 sequences up to 8192 / 2048 tokens, 8 x 128
+// bf16, 351 / 81.8 -> 296 / 77.2, E4M3 237 / 61.4 -> 234 / (63.5: below the
+// tile count); 16 sequences up to 8192 (24000 tiles) 34.5 -> 35.2, uniform
+// lengths (half the rows) 1570 -> 1628: those keep the smaller tiles.
+constexpr int64_t kRaggedSparse = 3;
+constexpr int64_t kRaggedSparseTiles = 49152;
 // RAGGED copies in gather_ragged_tile_kernel: two tiles per workgroup when a
 // sequence has kRaggedFoldMinUnits to kRaggedFoldMaxUnits tiles.  Against one tile per workgroup (same-box A/B, medians of 6
 // rounds, us per layer): c2's RAGGED gather 1563.7 -> 1528.0 (8 layers) and

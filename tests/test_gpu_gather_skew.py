@@ -1,5 +1,6 @@
-"""GPU parity of gathers whose grid mostly lies past the sequences: every
-table format with lengths of 0, negative, cut inside a tile and past max_seq_len."""
+"""GPU parity of gathers whose grid mostly lies past the sequences: RAGGED
+batches on both sides of the rule that doubles a tile's rows, and every table
+format with lengths of 0, negative, cut inside a tile and past max_seq_len."""
 import numpy as np
 import pytest
 import torch
@@ -13,6 +14,36 @@ from gpu_helpers import (TORCH_DT, OffsetsPool, check_gather, check_gather_offse
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 NHD, HND, PK = Layout.BLOCK_NHD, Layout.BLOCK_HND, Layout.BLOCK_HND_PACKED
+
+
+@pytest.mark.parametrize("extra", [-1, 0])
+def test_ragged_sparse_tiles(extra):
+    """49152 filled tiles of one 1552-byte row (the rule's least), or one
+    token fewer: whole blocks, blocks that change inside a doubled tile, and
+    skipped ids."""
+    rng = np.random.default_rng(5)
+    gen = torch.Generator().manual_seed(5)
+    H, D, bs, S = 1, 776, 16, 24
+    lens = np.full(S, 300)
+    lens[3] = 12000
+    lens[11] = 49152 + extra - lens[:11].sum() - lens[12:].sum()
+    L = int(lens.max())
+    assert lens.sum() == 49152 + extra and lens.sum() * 3 < S * L
+    nb = 3300
+    pc, kb, vb = make_cache(NHD, NHD, DType.BF16, nb, bs, H, D, gen=gen)
+    rows = [np.repeat(rng.integers(0, nb, size=-(-n // bs)), bs)[:n] for n in lens]
+    rows[3][::7] = nb - 2  # rows of a tile in different blocks
+    rows[5][::3] = -1
+    rows[6][:] = nb
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    table = paged.RaggedTable(torch.from_numpy(np.concatenate(rows).astype(np.int32)).to(DEV),
+                              torch.from_numpy(indptr).to(DEV))
+    ko = torch.zeros((S, L, H, D), dtype=torch.bfloat16, device=DEV)
+    vo = torch.zeros_like(ko)
+    dl = lens.copy()
+    dl[0], dl[1], dl[2], dl[4] = 0, -3, 77, L + 9
+    check_gather_ragged(pc, kb, vb, ko, vo, table, torch.from_numpy(dl.astype(np.int32)).to(DEV),
+                        L, cache_dtype=DType.BF16, io_dtype=DType.BF16)
 
 
 @pytest.mark.parametrize("fp8", [False, True])
