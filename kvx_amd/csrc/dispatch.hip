@@ -177,13 +177,17 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
                 int64_t *grid, uint32_t *lds_bytes) {
   const bool offsets = p.format == KVX_BLOCK_TABLE_KV_OFFSETS;
   const bool ragged = p.format == KVX_BLOCK_TABLE_RAGGED;
-  if (ragged && p.block_size > kTileMaxRows) return false;  // a tile's row ids in LDS
-  const int64_t bs = p.block_size;
+  // a block's rows, or those of one of its parts
+  const int64_t full_bs = p.block_size;
+  const int full_log2 = log2_exact(full_bs);
+  const int parts_log2 = full_log2 > kTileMaxRowsLog2 ? full_log2 - kTileMaxRowsLog2 : 0;
+  const int64_t bs = full_bs >> parts_log2;
   const int64_t H = p.heads;
   const int64_t D = p.head_dim;
   const int64_t row_cache = H * D * cs;
   const int bs_log2 = log2_exact(bs);
-  if (bs_log2 < 0 || row_cache < 16) return false;
+  if (full_log2 < 0 || row_cache < 16) return false;
+  if (row_cache * full_bs > 0x7FFFFFFF) return false;  // 32-bit offsets in a block
   const Geom *g[2] = {&p.gk, &p.gv};
   const void *src[2] = {p.src_k, p.src_v};
   void *dst[2] = {p.dst_k, p.dst_v};
@@ -193,7 +197,7 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
   int64_t min_tw = 16;
   int64_t unit = 16;  // a tile width holds whole runs and 16-byte chunks
   for (int i = 0; i < 2; ++i) {
-    const int64_t w = dense_run_elems(*g[i], bs, H, D);
+    const int64_t w = dense_run_elems(*g[i], full_bs, H, D);
     if (w < 0) return false;
     run_log2[i] = w == H * D ? -1 : log2_exact(w * cs);
     if (w != H * D) {
@@ -218,19 +222,6 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
     if (reinterpret_cast<uintptr_t>(dst[i]) % dst_align != 0) return false;
   }
   if (!transposed) return false;  // row-major pairs: the flat kernels
-  // RAGGED blocks of more rows than a wave has lanes load their row ids with
-  // every thread and one more barrier: taken where a tensor's runs are
-  // narrower than a 128-byte line (x-packed, token axis innermost), which
-  // the row kernel reads piece by piece.  On MI355X (c2's lengths, RAGGED,
-  // 128-token blocks, same-box A/B) x-packed K and V 2715 -> 1720 us,
-  // vLLM's pair 5455 -> 2019 us; HND (256-byte runs) 1640 -> 1718 us, so HND
-  // keeps the row kernel.
-  if (ragged && bs > kWave) {
-    int64_t narrow = -1;
-    for (int i = 0; i < 2; ++i)
-      if (run_bytes[i] > 0 && (narrow < 0 || run_bytes[i] < narrow)) narrow = run_bytes[i];
-    if (narrow >= 128) return false;
-  }
   if ((D * cs) % src_chunk != 0) return false;  // chunks never straddle heads
   // Tile width: a power of two that divides the row and holds whole runs.
   // A row that is not a power of two (6 or 12 heads, say) makes several
@@ -245,12 +236,8 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
     if (tw < 0) return false;
   } else {
     // halve toward kTileBytes, but not below one 128-byte output line per
-    // row (blocks of 128 or 256 tokens then take 16 or 32 KiB tiles): on
-    // MI355X (c2's lengths, bf16 x-packed blocks of 128 / 256 tokens) 2315 /
-    // 6752 -> 1789 / 1823 us per layer, where narrower rows split output
-    // lines between workgroups.  (Runs of whole lines, HND, also gathered
-    // faster in these tiles than in gather_rows_kernel at every block size
-    // that fits: 16-128 tokens, 4-12% at c2's size.)
+    // row: narrower rows split output lines between workgroups (x-packed
+    // blocks of 128 tokens in 64-byte tile rows 2315 -> 1789 us per layer)
     while (tw * bs > kTileBytes && tw / 2 >= min_tw && tw / 2 >= kTileMinWidth) tw /= 2;
   }
   const int64_t pitch = tw + kTilePad;
@@ -268,8 +255,8 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
   t->max_blocks_per_seq = p.max_blocks_per_seq;
   const int64_t by_len = ((int64_t)p.max_seq_len + bs - 1) / bs;
   // RAGGED rows do not use max_blocks_per_seq
-  t->blocks_per_seq = (int32_t)(ragged || by_len < p.max_blocks_per_seq ? by_len
-                                                                       : p.max_blocks_per_seq);
+  const int64_t by_table = (int64_t)p.max_blocks_per_seq << parts_log2;
+  t->blocks_per_seq = (int32_t)(ragged || by_len < by_table ? by_len : by_table);
   t->tiles = (int32_t)(row_cache / tw);
   t->tw = (int32_t)tw;
   t->tw_log2 = log2_exact(tw);
@@ -293,6 +280,7 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
   t->head_dim = p.head_dim;
   t->row_elems = (int32_t)(H * D);
   t->bs_log2 = bs_log2;
+  t->parts_log2 = parts_log2;
   t->cache_es_log2 = log2_exact(cs);
   t->io_es_log2 = log2_exact(is);
   const ScaleRef sc[2] = {p.k_scale, p.v_scale};
@@ -306,7 +294,11 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
     // for runs below 2^16 bytes
     t->t[i].run_bytes = (int32_t)run_bytes[i];
     t->t[i].run_magic = run_log2[i] == kRunOdd ? magic_for(run_bytes[i]) : 0;
-    t->t[i].pad_ = 0;
+    const int64_t run = run_log2[i] < 0 ? row_cache : run_bytes[i];
+    t->t[i].gap = run_log2[i] < 0 ? 0 : (int32_t)((full_bs - bs) * run);
+    if (t->t[i].gap >= 1 << 24 || row_cache / run >= 1 << 24) return false;
+    t->t[i].s_tile = tw * (run_log2[i] < 0 ? bs : full_bs);
+    t->t[i].s_part = bs * run;
   }
   *grid = (int64_t)p.seq_count * t->blocks_per_seq * t->tiles;
   *lds_bytes = (uint32_t)(bs * pitch);

@@ -1446,6 +1446,10 @@ __global__ __launch_bounds__(kBlockThreads) void gather_rows_kernel(GatherArgs a
 // sit at offsets 0 .. bs - 1 of their blocks, so a tile whose rows all name
 // one block is gathered like a PACKED one, and any other tile reads each
 // row's pieces from that row's block (the first wave compares the ids).
+//
+// Blocks of more than kTileMaxRows tokens are gathered in parts of that many:
+// a part's tile is `tw` cache bytes of its rows, whose runs lie `gap` bytes
+// further apart than the part's share of them.
 
 struct TileTensor {
   const char *src;    // cache tensor
@@ -1456,12 +1460,21 @@ struct TileTensor {
                       // kRunOdd: run_bytes, a multiple of 16 bytes
   int32_t run_bytes;
   uint32_t run_magic;  // kRunOdd: div_magic's m for run_bytes
-  int32_t pad_;
+  int32_t gap;         // bytes of the block between a tile's shares of two runs, < 2^24
+  int64_t s_tile;      // bytes of the block from tile to tile
+  int64_t s_part;      // ... and from part to part
 };
 
-// Rows of a tile (block_size) at most: the planner keeps
-// block_size * (tw + 16) within 64 KiB of LDS with tw >= 128.
-constexpr int kTileMaxRows = 256;
+// Rows of a tile at most: one wave's lanes.  Tiles of whole 128- and 256-token
+// blocks were 16 and 32 KiB, few of them resident per CU.  MI355X, 64000 tokens
+// of 8 x 128, us per gather, whole blocks (or the row kernels, where a tile
+// did not fit LDS) -> parts of 64: vLLM's pair bf16 in 128 / 256 / 512 tokens,
+// PACKED 108 / 170 / 578 -> 98 / 98 / 98, RAGGED 116 / 179 / 309 -> 96 / 97 /
+// 95; x-packed E4M3 78 / 88 / 103 -> 73 / 73 / 71; HND RAGGED E4M3 90 / 93 /
+// 92 -> 74 / 75 / 73; three heads HND 128 tokens RAGGED 46 -> 37, 256 tokens
+// PACKED 50 -> 38.
+constexpr int kTileMaxRowsLog2 = 6;
+constexpr int kTileMaxRows = 1 << kTileMaxRowsLog2;
 
 struct TileArgs {
   TileTensor t[2];
@@ -1486,7 +1499,8 @@ struct TileArgs {
   int32_t num_blocks;
   int32_t head_dim;
   int32_t row_elems;      // H * D
-  int32_t bs_log2;
+  int32_t bs_log2;        // of the tile's rows: a block's, or a part's
+  int32_t parts_log2;     // log2 parts per block
   int32_t cache_es_log2;  // log2 cache element bytes
   int32_t io_es_log2;     // log2 output element bytes
 };
@@ -1523,7 +1537,7 @@ __device__ __forceinline__ void put_piece(char *p, const Raw<16> &x, int k) {
 template <int PIECE>
 __device__ __forceinline__ void stage_tile(const char *region, char *lds, int32_t nbytes,
                                            int32_t run_log2, int32_t bs_log2, int32_t pitch,
-                                           int32_t rows) {
+                                           int32_t rows, int32_t gap) {
   const int32_t bsm = (1 << bs_log2) - 1;
   const int32_t runm = (1 << run_log2) - 1;
   const int32_t kStep = (int32_t)blockDim.x * 16;
@@ -1533,7 +1547,7 @@ __device__ __forceinline__ void stage_tile(const char *region, char *lds, int32_
     for (int u = 0; u < kTileLoads; ++u) {
       const int32_t m = m0 + u * kStep;
       if (m < nbytes && ((m >> run_log2) & bsm) < rows)
-        x[u] = ld<16, kGatherNtLoad>(region + m);
+        x[u] = ld<16, kGatherNtLoad>(region + m + __umul24(m >> (run_log2 + bs_log2), gap));
     }
 #pragma unroll
     for (int u = 0; u < kTileLoads; ++u) {
@@ -1555,10 +1569,10 @@ __device__ __forceinline__ void stage_tile(const char *region, char *lds, int32_
 // is loaded from its own row's block, ids[o] (< 0: row skipped); `off` is
 // the tile's region offset within a block.
 template <int PIECE>
-__device__ __forceinline__ void stage_tile_rows(const char *src, int64_t s_block, int32_t off,
+__device__ __forceinline__ void stage_tile_rows(const char *src, int64_t s_block, int64_t off,
                                                 const int64_t *ids, char *lds, int32_t nbytes,
                                                 int32_t run_log2, int32_t bs_log2, int32_t pitch,
-                                                int32_t rows) {
+                                                int32_t rows, int32_t gap) {
   const int32_t bsm = (1 << bs_log2) - 1;
   const int32_t runm = (1 << run_log2) - 1;
   for (int32_t mm = (int32_t)threadIdx.x * PIECE; mm < nbytes; mm += (int32_t)blockDim.x * PIECE) {
@@ -1568,7 +1582,7 @@ __device__ __forceinline__ void stage_tile_rows(const char *src, int64_t s_block
     if (id < 0) continue;
     const int32_t ar = mm >> (run_log2 + bs_log2);
     st<PIECE>(lds + o * pitch + (ar << run_log2) + (mm & runm),
-              ld<PIECE, kGatherNtLoad>(src + id * s_block + off + mm));
+              ld<PIECE, kGatherNtLoad>(src + id * s_block + off + mm + __umul24(ar, gap)));
   }
 }
 
@@ -1577,7 +1591,7 @@ __device__ __forceinline__ void stage_tile_rows(const char *src, int64_t s_block
 // multiply-high) gives the row (index % bs) and the run's place in the row.
 __device__ __forceinline__ void stage_tile_odd(const char *region, char *lds, int32_t nbytes,
                                                int32_t run, uint32_t run_magic, int32_t bs_log2,
-                                               int32_t pitch, int32_t rows) {
+                                               int32_t pitch, int32_t rows, int32_t gap) {
   const uint32_t bsm = (1u << bs_log2) - 1;
   const int32_t kStep = (int32_t)blockDim.x * 16;
   for (int32_t m0 = (int32_t)threadIdx.x * 16; m0 < nbytes; m0 += kTileLoads * kStep) {
@@ -1592,7 +1606,7 @@ __device__ __forceinline__ void stage_tile_odd(const char *region, char *lds, in
         const int32_t o = (int32_t)(q & bsm);
         if (o < rows) {
           at[u] = o * pitch + (int32_t)(q >> bs_log2) * run + (m - (int32_t)q * run);
-          x[u] = ld<16, kGatherNtLoad>(region + m);
+          x[u] = ld<16, kGatherNtLoad>(region + m + __umul24(q >> bs_log2, gap));
         }
       }
     }
@@ -1604,10 +1618,11 @@ __device__ __forceinline__ void stage_tile_odd(const char *region, char *lds, in
 
 // stage_tile_rows for runs of `run` bytes (a multiple of 16, not a power of
 // two): 16-byte pieces, each inside one run.
-__device__ __forceinline__ void stage_tile_rows_odd(const char *src, int64_t s_block, int32_t off,
+__device__ __forceinline__ void stage_tile_rows_odd(const char *src, int64_t s_block, int64_t off,
                                                     const int64_t *ids, char *lds, int32_t nbytes,
                                                     int32_t run, uint32_t run_magic,
-                                                    int32_t bs_log2, int32_t pitch, int32_t rows) {
+                                                    int32_t bs_log2, int32_t pitch, int32_t rows,
+                                                    int32_t gap) {
   const uint32_t bsm = (1u << bs_log2) - 1;
   for (int32_t mm = (int32_t)threadIdx.x * 16; mm < nbytes; mm += (int32_t)blockDim.x * 16) {
     const uint32_t q = div_magic((uint32_t)mm, run_magic);
@@ -1616,7 +1631,7 @@ __device__ __forceinline__ void stage_tile_rows_odd(const char *src, int64_t s_b
     const int64_t id = ids[o];
     if (id < 0) continue;
     st<16>(lds + o * pitch + (int32_t)(q >> bs_log2) * run + (mm - (int32_t)q * run),
-           ld<16, kGatherNtLoad>(src + id * s_block + off + mm));
+           ld<16, kGatherNtLoad>(src + id * s_block + off + mm + __umul24(q >> bs_log2, gap)));
   }
 }
 
@@ -1709,57 +1724,41 @@ __global__ __launch_bounds__(kBlockThreads) void gather_tiles_kernel(TileArgs a)
     if (t0 >= n) return;
     const int64_t rem = n - t0;
     const int32_t rws = rem < bs ? (int32_t)rem : bs;
-    if (bs <= kWave) {
-      // one wave loads the ids, one per lane, and a ballot compares them
-      if (threadIdx.x < kWave) {
-        const int lane = (int)threadIdx.x;
-        int64_t id = -1;
-        if (lane < rws) {
-          id = load_idx<I64>(a.table, start + t0 + lane);
-          if (id < 0 || id >= a.num_blocks) id = -1;
-          s_ids[lane] = id;
-        }
-        const int64_t first =
-            (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(id >> 32))
-                       << 32) |
-                      (uint32_t)__builtin_amdgcn_readfirstlane((int)id));
-        const uint64_t same = __ballot(lane >= rws || id == first);
-        if (lane == 0) s_same = same == ~0ull;
-      }
-      __syncthreads();
-      bid = s_ids[0];
-      mixed = !s_same;
-    } else {
-      // blocks of more rows than a wave has lanes: every thread loads ids,
-      // then a barrier that ORs the threads' mismatches with row 0's id
-      for (int32_t r = (int32_t)threadIdx.x; r < rws; r += (int32_t)blockDim.x) {
-        int64_t id = load_idx<I64>(a.table, start + t0 + r);
+    // one wave loads the ids, one per lane, and a ballot compares them
+    if (threadIdx.x < kWave) {
+      const int lane = (int)threadIdx.x;
+      int64_t id = -1;
+      if (lane < rws) {
+        id = load_idx<I64>(a.table, start + t0 + lane);
         if (id < 0 || id >= a.num_blocks) id = -1;
-        s_ids[r] = id;
+        s_ids[lane] = id;
       }
-      __syncthreads();
-      bid = s_ids[0];
-      int differs = 0;
-      for (int32_t r = (int32_t)threadIdx.x; r < rws; r += (int32_t)blockDim.x)
-        differs |= s_ids[r] != bid;
-      mixed = __syncthreads_or(differs) != 0;
+      const int64_t first =
+          (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(id >> 32)) << 32) |
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)id));
+      const uint64_t same = __ballot(lane >= rws || id == first);
+      if (lane == 0) s_same = same == ~0ull;
     }
+    __syncthreads();
+    bid = s_ids[0];
+    mixed = !s_same;
     if (!mixed) {
       if (bid < 0) return;  // every row skipped
       blk = tt.src + bid * tt.s_block;
     }
   } else {
-    if (lb >= a.max_blocks_per_seq) return;
+    const int32_t blb = lb >> a.parts_log2;  // the part's block of the sequence
+    if (blb >= a.max_blocks_per_seq) return;
     if constexpr (FMT == KVX_BLOCK_TABLE_KV_OFFSETS) {
       // table [seq, beam = 1, {K, V}, max_blocks_per_seq] of KVCacheIndex
       const uint32_t ent = reinterpret_cast<const uint32_t *>(
-          a.table)[(s * 2 + blockIdx.y) * a.max_blocks_per_seq + lb];
+          a.table)[(s * 2 + blockIdx.y) * a.max_blocks_per_seq + blb];
       const char *pool = (ent >> 31) ? a.pool[1] : a.pool[0];
       bid = ent & 0x7FFFFFFFu;
       if (pool == nullptr || bid >= ((ent >> 31) ? a.pool_blocks[1] : a.pool_blocks[0])) return;
       blk = pool + bid * a.bytes_per_block;
     } else {
-      bid = load_idx<I64>(a.table, s * a.max_blocks_per_seq + lb);
+      bid = load_idx<I64>(a.table, s * a.max_blocks_per_seq + blb);
       if (bid < 0 || bid >= a.num_blocks) return;
       blk = tt.src + bid * tt.s_block;
     }
@@ -1774,6 +1773,8 @@ __global__ __launch_bounds__(kBlockThreads) void gather_tiles_kernel(TileArgs a)
   char *out = tt.dst + (s * a.max_seq_len + t0) * a.out_row_bytes;
   const uint32_t hd = (uint32_t)a.head_dim;
   const uint32_t re = (uint32_t)a.row_elems;
+
+  const int64_t part = (int64_t)(lb & ((1 << a.parts_log2) - 1)) * tt.s_part;
 
   if (tt.run_log2 < 0) {
     // Row-major block: rows are contiguous in the cache and in the output.
@@ -1794,33 +1795,34 @@ __global__ __launch_bounds__(kBlockThreads) void gather_tiles_kernel(TileArgs a)
       float sc = uniform;
       if constexpr (Op::kScaled) sc = scale_in_rows(tt.sc, uniform, rb, e, re, hd);
       st<Op::kDst, kGatherNtStore>(out + ((int64_t)e << a.io_es_log2),
-                                   Op::apply(ld<Op::kSrc, kGatherNtLoad>(b + m), sc));
+                                   Op::apply(ld<Op::kSrc, kGatherNtLoad>(b + part + m), sc));
     }
     return;
   }
 
   if (mixed) {
-    const int32_t off = tile * region;
+    const int64_t off = part + tile * tt.s_tile;
     if (tt.run_log2 == kRunOdd)
       stage_tile_rows_odd(tt.src, tt.s_block, off, s_ids, lds, region, tt.run_bytes, tt.run_magic,
-                          a.bs_log2, a.pitch, rows);
+                          a.bs_log2, a.pitch, rows, tt.gap);
     else switch (tt.run_log2) {
-      case 0: stage_tile_rows<1>(tt.src, tt.s_block, off, s_ids, lds, region, 0, a.bs_log2, a.pitch, rows); break;
-      case 1: stage_tile_rows<2>(tt.src, tt.s_block, off, s_ids, lds, region, 1, a.bs_log2, a.pitch, rows); break;
-      case 2: stage_tile_rows<4>(tt.src, tt.s_block, off, s_ids, lds, region, 2, a.bs_log2, a.pitch, rows); break;
-      case 3: stage_tile_rows<8>(tt.src, tt.s_block, off, s_ids, lds, region, 3, a.bs_log2, a.pitch, rows); break;
-      default: stage_tile_rows<16>(tt.src, tt.s_block, off, s_ids, lds, region, tt.run_log2, a.bs_log2, a.pitch, rows); break;
+      case 0: stage_tile_rows<1>(tt.src, tt.s_block, off, s_ids, lds, region, 0, a.bs_log2, a.pitch, rows, tt.gap); break;
+      case 1: stage_tile_rows<2>(tt.src, tt.s_block, off, s_ids, lds, region, 1, a.bs_log2, a.pitch, rows, tt.gap); break;
+      case 2: stage_tile_rows<4>(tt.src, tt.s_block, off, s_ids, lds, region, 2, a.bs_log2, a.pitch, rows, tt.gap); break;
+      case 3: stage_tile_rows<8>(tt.src, tt.s_block, off, s_ids, lds, region, 3, a.bs_log2, a.pitch, rows, tt.gap); break;
+      default: stage_tile_rows<16>(tt.src, tt.s_block, off, s_ids, lds, region, tt.run_log2, a.bs_log2, a.pitch, rows, tt.gap); break;
     }
   } else {
-    const char *src = blk + (int64_t)tile * region;
+    const char *src = blk + part + tile * tt.s_tile;
     if (tt.run_log2 == kRunOdd)
-      stage_tile_odd(src, lds, region, tt.run_bytes, tt.run_magic, a.bs_log2, a.pitch, rows);
+      stage_tile_odd(src, lds, region, tt.run_bytes, tt.run_magic, a.bs_log2, a.pitch, rows,
+                     tt.gap);
     else switch (tt.run_log2) {
-      case 0: stage_tile<1>(src, lds, region, 0, a.bs_log2, a.pitch, rows); break;
-      case 1: stage_tile<2>(src, lds, region, 1, a.bs_log2, a.pitch, rows); break;
-      case 2: stage_tile<4>(src, lds, region, 2, a.bs_log2, a.pitch, rows); break;
-      case 3: stage_tile<8>(src, lds, region, 3, a.bs_log2, a.pitch, rows); break;
-      default: stage_tile<16>(src, lds, region, tt.run_log2, a.bs_log2, a.pitch, rows); break;
+      case 0: stage_tile<1>(src, lds, region, 0, a.bs_log2, a.pitch, rows, tt.gap); break;
+      case 1: stage_tile<2>(src, lds, region, 1, a.bs_log2, a.pitch, rows, tt.gap); break;
+      case 2: stage_tile<4>(src, lds, region, 2, a.bs_log2, a.pitch, rows, tt.gap); break;
+      case 3: stage_tile<8>(src, lds, region, 3, a.bs_log2, a.pitch, rows, tt.gap); break;
+      default: stage_tile<16>(src, lds, region, tt.run_log2, a.bs_log2, a.pitch, rows, tt.gap); break;
     }
   }
   __syncthreads();
