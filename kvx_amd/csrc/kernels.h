@@ -832,13 +832,7 @@ __global__ __launch_bounds__(kBlockThreads) void write_tiles_kernel(WriteTileArg
   const int32_t lane = tid & (kWave - 1);
   const int32_t nt = (int32_t)blockDim.x;
 
-  // Lane l holds the slot of row l - lane0 of the tile (narrow: from the row
-  // before it to the rows that may follow it).
   const int32_t lane0 = t.align > 1 ? 1 : 0;
-  const int64_t ts = t0 + lane - lane0;
-  int64_t slot = -1;
-  if (ts >= 0 && ts < a.num_tokens && lane < t.rows + lane0 * t.align)
-    slot = load_index(a.slots, ts, a.slot_is64);
   // chunk u is chunk u % cpr of row u / cpr
   const int32_t total = left * t.cpr;
   const char *src = t.src + t0 * a.row_bytes + (int64_t)tile * t.cpr * Op::kSrc;
@@ -852,6 +846,14 @@ __global__ __launch_bounds__(kBlockThreads) void write_tiles_kernel(WriteTileArg
       x[k] = ld<Op::kSrc, kWriteNtLoad>(src + row[k] * a.row_bytes +
                                         (int64_t)(u - row[k] * t.cpr) * Op::kSrc);
   }
+  // Lane l holds the slot of row l - lane0 of the tile (narrow: from the row
+  // before it to the rows that may follow it).  Loaded behind the rows, whose
+  // addresses do not need it: 32768 tokens of 8 x 128 bf16 into x-packed K
+  // and NHD V 53.7 -> 53.1 us.
+  const int64_t ts = t0 + lane - lane0;
+  int64_t slot = -1;
+  if (ts >= 0 && ts < a.num_tokens && lane < t.rows + lane0 * t.align)
+    slot = load_index(a.slots, ts, a.slot_is64);
   float uniform = 1.0f;
   if constexpr (Op::kScaled) uniform = t.sc.p[0];
 
