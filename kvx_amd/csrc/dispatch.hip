@@ -701,11 +701,13 @@ kvx_status_t enqueue_gather(const GatherPlan &p, void *stream) {
     // rows.  Rows that are H*D contiguous elements (any row stride) take the
     // flat kernels, which find a chunk's row by a shift or, for chunk counts
     // that are not a power of two (DeepSeek's 576-element MLA rows: 72), by
-    // a multiply-high, exact while tile chunks * nchunks <= 2^32 (so at most
-    // 1024 chunks per row there); otherwise the row kernel, with at least
+    // a multiply-high, exact while tile chunks * nchunks <= 2^32, for rows of
+    // at most kFlatRowChunks chunks; otherwise the row kernel, with at least
     // one full pass of its row groups.
     auto row_dense = [&](const Geom &g) { return row_elems_contiguous(g, p.head_dim, p.heads); };
-    const bool chunks_ok = a.nchunks_log2 >= 0 || a.nchunks <= 1024;
+    const int max_chunks =
+        p.conv == kConvDequant && is == 4 ? kFlatRowChunksDequantF32 : kFlatRowChunks;
+    const bool chunks_ok = a.nchunks_log2 >= 0 || a.nchunks <= max_chunks;
     a.flat = row_dense(p.gk) && row_dense(p.gv) && chunks_ok;
     if (ragged_tile && chunks_ok) {
       // R rows of about kFlatTileBytes of cache per tensor: a power of

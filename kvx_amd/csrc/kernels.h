@@ -101,6 +101,16 @@ constexpr int64_t kRaggedCopyTileBytes = 2048;
 // Chunks per thread the RAGGED / KV_OFFSETS flat gather resolves and loads
 // together (the table load and the data load of each are dependent).
 constexpr int kIndexedUnroll = 4;
+// Rows of a chunk count that is not a power of two take the RAGGED / KV_OFFSETS
+// flat gathers up to kFlatRowChunks chunks (16-byte ones: 8192 bf16 elements).
+// Wider rows gain 7-10% in back-to-back gathers there and lose up to 6% where
+// the cache is cold (24 sequences of up to 1024 rows of 72 x 128 bf16, padded
+// rows, RAGGED, us: 264 -> 258, cold 245 -> 261), so they keep the row kernel.
+// Four-code chunks into f32 hold the same rows in twice the count: 40 x 128,
+// E4M3 to f32, in the row kernel -> here: RAGGED 214 -> 171, KV_OFFSETS 221 ->
+// 166; 48 x 128 254 -> 206 and 258 -> 201.
+constexpr int kFlatRowChunks = 1024;
+constexpr int kFlatRowChunksDequantF32 = 2048;
 // KV_OFFSETS row-dense gather: the dequantizing gather loads its table
 // entries once per workgroup tile (per-chunk loads cost it, with 8-byte
 // source chunks and twice the table loads per byte, 15%).  The copy gather

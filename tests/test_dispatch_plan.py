@@ -1,0 +1,20 @@
+"""Which kernel the launch planning picks, and its shape, at the rules'
+edges, on the CPU (tests/dispatch_plan.py)."""
+import pytest
+
+import dispatch_plan as dp
+from kvx_amd.abi import DType, Layout
+
+NHD, HND, PK = Layout.BLOCK_NHD, Layout.BLOCK_HND, Layout.BLOCK_HND_PACKED
+BF16, F32, E4M3, E5M2 = DType.BF16, DType.F32, DType.F8_E4M3, DType.F8_E5M2
+
+
+@pytest.mark.parametrize("table,flat", [("ragged", "gather_ragged_tile"),
+                                        ("offsets", "gather_indexed_flat")])
+def test_wide_rows_into_f32_stay_in_the_flat_gathers(table, flat):
+    for H in (33, 40, 63):  # 4224 to 8064 elements, in chunks of four
+        assert dp.gather(NHD, table, E4M3, F32, 16, H, 128)["kernel"] == flat
+    assert dp.gather(NHD, table, E4M3, F32, 16, 72, 128)["kernel"] == "gather_indexed"
+    for io, H, kernel in ((BF16, 63, flat), (BF16, 72, "gather_indexed")):
+        assert dp.gather(NHD, table, E4M3, io, 16, H, 128)["kernel"] == kernel
+        assert dp.gather(NHD, table, io, io, 16, H, 128)["kernel"] == kernel

@@ -57,3 +57,32 @@ def test_gather_into_f32(shape, layout, table):
     check_gather_ragged(pc, kb, vb, ko, vo,
                         paged.RaggedTable(torch.from_numpy(rows.reshape(-1)).to(DEV),
                                           torch.from_numpy(indptr).to(DEV)), lens, L, **kw)
+
+
+@pytest.mark.parametrize("table", ["ragged", "offsets"])
+@pytest.mark.parametrize("heads", [40, 63])
+def test_wide_rows(heads, table):
+    """Rows of 1280 and 2016 four-code chunks, in the flat indexed gathers."""
+    D, bs, nb, S, L = 128, 16, 12, 3, 45
+    rng = np.random.default_rng(heads)
+    gen = torch.Generator().manual_seed(heads)
+    scales = [ScaleArg(SG.PER_HEAD, rng.uniform(0.01, 0.05, heads)) for _ in range(2)]
+    lens = torch.tensor([L, bs + 1, L + 7], dtype=torch.int32, device=DEV)
+    ko = random_fill(torch.empty((S, L, heads, D), dtype=torch.float32, device=DEV), gen)
+    vo = random_fill(torch.empty_like(ko), gen)
+    kw = dict(cache_dtype=DType.F8_E4M3, io_dtype=DType.F32, k_scale=scales[0], v_scale=scales[1])
+    if table == "offsets":
+        pool = OffsetsPool(NHD, NHD, DType.F8_E4M3, nb, bs, heads, D, pitch_pad=16, gen=gen)
+        raw = rng.integers(0, nb + 1, size=(S, 1, 2, 3)).astype(np.uint32)
+        raw |= (rng.random(raw.shape) < 0.3).astype(np.uint32) << 31
+        check_gather_offsets(pool, ko, vo, torch.from_numpy(raw.view(np.int32)).to(DEV), lens, L,
+                             **kw)
+        return
+    pc, kb, vb = make_cache(NHD, NHD, DType.F8_E4M3, nb, bs, heads, D, gen=gen)
+    rows = np.repeat(rng.integers(-1, nb + 1, size=(S, 3)).astype(np.int32), bs, axis=1)[:, :L]
+    rows = rows.copy()
+    rows[1, ::5] = nb - 1
+    indptr = np.arange(S + 1, dtype=np.int32) * L
+    check_gather_ragged(pc, kb, vb, ko, vo,
+                        paged.RaggedTable(torch.from_numpy(rows.reshape(-1)).to(DEV),
+                                          torch.from_numpy(indptr).to(DEV)), lens, L, **kw)
