@@ -22,6 +22,14 @@ std::string field(const char *name, int64_t v) {
 
 extern "C" const char *kvx_plan() { return g_plan.c_str(); }
 
+// Chunks in flight of the flat dequantizing gathers of `codes` codes.
+extern "C" int kvx_flat_unroll(int codes, int f32) {
+  using namespace kvx::dev;
+  if (f32) return flat_unroll<DequantOp<4, KVX_DTYPE_F32, KVX_DTYPE_F8_E4M3>>();
+  return codes == 4 ? flat_unroll<DequantOp<4, KVX_DTYPE_BF16, KVX_DTYPE_F8_E4M3>>()
+                    : flat_unroll<DequantOp<8, KVX_DTYPE_BF16, KVX_DTYPE_F8_E4M3>>();
+}
+
 namespace kvx {
 namespace dev {
 namespace {

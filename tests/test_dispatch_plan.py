@@ -18,3 +18,8 @@ def test_wide_rows_into_f32_stay_in_the_flat_gathers(table, flat):
     for io, H, kernel in ((BF16, 63, flat), (BF16, 72, "gather_indexed")):
         assert dp.gather(NHD, table, E4M3, io, 16, H, 128)["kernel"] == kernel
         assert dp.gather(NHD, table, io, io, 16, H, 128)["kernel"] == kernel
+
+
+def test_four_code_chunks_in_flight():
+    unroll = dp.lib().kvx_flat_unroll
+    assert (unroll(4, True), unroll(4, False), unroll(8, False)) == (4, 2, 2)
