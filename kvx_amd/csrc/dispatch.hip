@@ -229,9 +229,12 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
   // on MI355X (c2's table) HND gathers of 6 x 128 and 12 x 64 bf16 heads
   // measured 0.676 of peak in 8 KiB tiles against 0.63 in gather_rows_kernel,
   // 3 x 128 heads 0.587 in 4 KiB tiles against 0.623.
+  // (The whole block counts there: parts of 64 rows keep the width, in smaller
+  // tiles, rather than take one that splits lines.  576-byte FP8 rows, x-packed,
+  // 128 / 256-token blocks, 180000 tokens: 64-byte tiles 111 us, 144-byte 186.)
   int64_t tw = row_cache & -row_cache;
   if (odd_run || tw < min_tw ||
-      ((row_cache & (row_cache - 1)) != 0 && tw * bs < kTileBytes)) {
+      ((row_cache & (row_cache - 1)) != 0 && tw * full_bs < kTileBytes)) {
     tw = odd_tile_width(row_cache, unit, bs, kTileBytes);
     if (tw < 0) return false;
   } else {

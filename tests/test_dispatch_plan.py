@@ -23,3 +23,12 @@ def test_wide_rows_into_f32_stay_in_the_flat_gathers(table, flat):
 def test_four_code_chunks_in_flight():
     unroll = dp.lib().kvx_flat_unroll
     assert (unroll(4, True), unroll(4, False), unroll(8, False)) == (4, 2, 2)
+
+
+@pytest.mark.parametrize("table", ["packed", "ragged", "offsets"])
+def test_parts_keep_the_tile_width_of_whole_blocks(table):
+    """576-byte rows: 64-byte tiles fill 8 KiB in blocks of 128 tokens and
+    more; in 64-token blocks they do not."""
+    for bs, tw in ((64, 144), (128, 64), (256, 64)):
+        plan = dp.gather(PK, table, E4M3, BF16, bs, 1, 576)
+        assert (plan["kernel"], plan["rows"], plan["tw"]) == ("gather_tiles", 64, tw)

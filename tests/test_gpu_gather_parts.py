@@ -72,3 +72,10 @@ def test_gather(layout, shape, table, bs, kind):
     check_gather_ragged(pc, kb, vb, ko, vo,
                         paged.RaggedTable(torch.from_numpy(rows.reshape(-1)).to(DEV),
                                           torch.from_numpy(indptr).to(DEV)), ld, L, **kw)
+
+
+@pytest.mark.parametrize("bs", [128, 256])
+@pytest.mark.parametrize("table", ["packed", "ragged", "offsets"])
+def test_parts_of_odd_rows(table, bs):
+    """576-byte rows: 64-byte tiles of 64 rows."""
+    test_gather("packed", (1, 576), table, bs, "e4m3")
