@@ -177,10 +177,23 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
                 int64_t *grid, uint32_t *lds_bytes) {
   const bool offsets = p.format == KVX_BLOCK_TABLE_KV_OFFSETS;
   const bool ragged = p.format == KVX_BLOCK_TABLE_RAGGED;
-  // a block's rows, or those of one of its parts
+  // a block's rows, or those of one of its parts.  Of 1-byte runs (a
+  // token-innermost FP8 tensor) 64 rows are half a line of every run, so parts
+  // hold 128 there, but for rows of a whole number of KiB (8, 16 and 24 heads of
+  // 128), which 64 suit better.  vLLM's pair, 128-token blocks, PACKED, E4M3
+  // to bf16, 180000 tokens, 64 -> 128 rows, us: 2 x 128 59.7 -> 54.8, 8 x 96 171
+  // -> 160, 12 x 128 348 -> 318, 576 (64-byte tiles) 127 -> 110; 8 x 128 202 ->
+  // 212, 24 x 128 617 -> 631.  RAGGED loads a
+  // part's block ids with one wave.
   const int64_t full_bs = p.block_size;
   const int full_log2 = log2_exact(full_bs);
-  const int parts_log2 = full_log2 > kTileMaxRowsLog2 ? full_log2 - kTileMaxRowsLog2 : 0;
+  const int64_t row_codes = (int64_t)p.heads * p.head_dim;
+  int part_rows_log2 = kTileMaxRowsLog2;
+  if (!ragged && cs == 1 && row_codes % 1024 != 0)
+    for (const Geom *t : {&p.gk, &p.gv})
+      if (dense_run_elems(*t, full_bs, p.heads, p.head_dim) == 1)
+        part_rows_log2 = kTileMaxRowsLog2 + 1;
+  const int parts_log2 = full_log2 > part_rows_log2 ? full_log2 - part_rows_log2 : 0;
   const int64_t bs = full_bs >> parts_log2;
   const int64_t H = p.heads;
   const int64_t D = p.head_dim;

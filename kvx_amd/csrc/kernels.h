@@ -1481,7 +1481,8 @@ struct TileTensor {
   int64_t s_part;      // ... and from part to part
 };
 
-// Rows of a tile at most: one wave's lanes.  Tiles of whole 128- and 256-token
+// Rows of a tile at most: one wave's lanes (twice that for some tensors of
+// 1-byte runs, see plan_tiles).  Tiles of whole 128- and 256-token
 // blocks were 16 and 32 KiB, few of them resident per CU.  MI355X, 64000 tokens
 // of 8 x 128, us per gather, whole blocks (or the row kernels, where a tile
 // did not fit LDS) -> parts of 64: vLLM's pair bf16 in 128 / 256 / 512 tokens,

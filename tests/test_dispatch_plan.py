@@ -32,3 +32,23 @@ def test_parts_keep_the_tile_width_of_whole_blocks(table):
     for bs, tw in ((64, 144), (128, 64), (256, 64)):
         plan = dp.gather(PK, table, E4M3, BF16, bs, 1, 576)
         assert (plan["kernel"], plan["rows"], plan["tw"]) == ("gather_tiles", 64, tw)
+
+
+def test_parts_of_one_byte_runs_hold_whole_lines():
+    """128 rows a part of a token-innermost FP8 tensor, unless its rows are a
+    whole number of KiB; the other formats and dtypes keep 64."""
+    def rows(cache, table, H, D, bs, io=BF16):
+        plan = dp.gather(dp.VLLM, table, cache, io, bs, H, D)
+        assert plan["kernel"] == "gather_tiles" and plan["rows"] * plan["parts"] == bs
+        return plan["rows"]
+
+    for bs in (128, 256, 512):
+        for H, D in ((1, 128), (2, 128), (8, 64), (8, 96), (1, 576), (12, 128)):
+            assert rows(E4M3, "packed", H, D, bs) == 128
+            assert rows(E5M2, "packed", H, D, bs, F32) == 128
+            assert rows(E4M3, "ragged", H, D, bs) == 64
+            assert rows(BF16, "packed", H, D, bs) == 64
+        for H, D in ((8, 128), (16, 128), (24, 128)):
+            assert rows(E4M3, "packed", H, D, bs) == 64
+    assert rows(E4M3, "packed", 2, 128, 64) == 64
+    assert dp.gather(PK, "packed", E4M3, BF16, 256, 2, 128)["rows"] == 64

@@ -79,3 +79,10 @@ def test_gather(layout, shape, table, bs, kind):
 def test_parts_of_odd_rows(table, bs):
     """576-byte rows: 64-byte tiles of 64 rows."""
     test_gather("packed", (1, 576), table, bs, "e4m3")
+
+
+@pytest.mark.parametrize("kind", ["e4m3", "e5m2 to f32"])
+@pytest.mark.parametrize("shape", [(1, 576), (8, 128)])
+def test_parts_of_one_byte_runs(shape, kind):
+    """vLLM's FP8 pair, PACKED, in parts of 128 rows and (8 x 128) of 64."""
+    test_gather("vllm", shape, "packed", 256, kind)
