@@ -183,8 +183,7 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
   // 128), which 64 suit better.  vLLM's pair, 128-token blocks, PACKED, E4M3
   // to bf16, 180000 tokens, 64 -> 128 rows, us: 2 x 128 59.7 -> 54.8, 8 x 96 171
   // -> 160, 12 x 128 348 -> 318, 576 (64-byte tiles) 127 -> 110; 8 x 128 202 ->
-  // 212, 24 x 128 617 -> 631.  RAGGED loads a
-  // part's block ids with one wave.
+  // 212, 24 x 128 617 -> 631.  RAGGED loads a part's block ids with one wave.
   const int64_t full_bs = p.block_size;
   const int full_log2 = log2_exact(full_bs);
   const int64_t row_codes = (int64_t)p.heads * p.head_dim;
@@ -235,6 +234,28 @@ bool plan_tiles(const GatherPlan &p, int cs, int is, int src_chunk, TileArgs *t,
     if (reinterpret_cast<uintptr_t>(dst[i]) % dst_align != 0) return false;
   }
   if (!transposed) return false;  // row-major pairs: the flat kernels
+  // Copies of whole-line runs (HND) through RAGGED and KV_OFFSETS tables keep
+  // gather_indexed_kernel where a whole block makes no tile (RAGGED: in any
+  // block of parts), its waves are full (a power of two of 16-byte chunks a
+  // row, or 64 and more) and its lanes hold a row's chunks (4 KiB; 3 KiB of
+  // runs of more than 256 bytes).  Parts -> rows, us, 36000 tokens back to
+  // back / cold / 180000 tokens, 256-token blocks: 8 x 128 bf16 RAGGED 53 / 59 /
+  // 252 -> 42 / 46 / 250, KV_OFFSETS 51 / 59 / 251 -> 41 / 43 / 232; 2 x 128 f32
+  // RAGGED 30 / 35 / 129 -> 22 / 28 / 130; 8 x 96 bf16 KV_OFFSETS 41 / 46 / 202
+  // -> 27 / 38 / 192.  Left in parts: 3 x 128 bf16 RAGGED 22 / 26 / 92 (rows 19 /
+  // 30 / 116), 8 x 128 f32 99 / 102 / 468 (117 / 97 / 546), 16 x 128 f32 190 /
+  // 192 / 930 (234 / 211 / 1120).
+  if (parts_log2 > 0 && p.conv == kConvCopy && (ragged || offsets)) {
+    int64_t narrowest = row_cache;
+    for (int i = 0; i < 2; ++i)
+      if (run_bytes[i] > 0 && run_bytes[i] < narrowest) narrowest = run_bytes[i];
+    const int64_t chunks = row_cache / 16;
+    const bool full_waves = log2_exact(chunks) >= 0 || chunks >= kWave;
+    const bool block_tile = !ragged && !odd_run && full_bs * (min_tw + kTilePad) <= 64 * 1024;
+    if (narrowest >= 128 && row_cache <= (narrowest > 256 ? 3072 : 4096) && full_waves &&
+        !block_tile)
+      return false;
+  }
   if ((D * cs) % src_chunk != 0) return false;  // chunks never straddle heads
   // Tile width: a power of two that divides the row and holds whole runs.
   // A row that is not a power of two (6 or 12 heads, say) makes several

@@ -52,3 +52,27 @@ def test_parts_of_one_byte_runs_hold_whole_lines():
             assert rows(E4M3, "packed", H, D, bs) == 64
     assert rows(E4M3, "packed", 2, 128, 64) == 64
     assert dp.gather(PK, "packed", E4M3, BF16, 256, 2, 128)["rows"] == 64
+
+
+def test_copies_of_whole_line_runs_in_big_blocks():
+    """RAGGED / KV_OFFSETS copies of HND blocks of more than 64 tokens: the
+    row kernel, or parts where its waves or registers do not suit the row."""
+    def kernel(table, H, D, bs, dtype=BF16, io=None):
+        return dp.gather(HND, table, dtype, io or dtype, bs, H, D)["kernel"]
+
+    rows, tiles = "gather_indexed", "gather_tiles"
+    for bs in (128, 256, 512):
+        for H, D, dt in ((2, 128, BF16), (8, 64, BF16), (8, 128, BF16), (16, 128, BF16),
+                         (6, 128, BF16), (8, 96, BF16), (2, 128, F32), (6, 128, F32)):
+            assert kernel("ragged", H, D, bs, dt) == rows
+            # KV_OFFSETS: a whole block whose tile fits 64 KiB goes in parts
+            run = D * (4 if dt == F32 else 2)
+            whole = D != 96 and bs * (run + 16) <= 65536
+            assert kernel("offsets", H, D, bs, dt) == (tiles if whole else rows)
+        for H, D, dt in ((3, 128, BF16), (8, 128, F32), (16, 128, F32)):
+            assert kernel("ragged", H, D, bs, dt) == tiles
+            assert kernel("offsets", H, D, bs, dt) == tiles
+        assert kernel("ragged", 8, 128, bs, E4M3, BF16) == tiles
+        assert dp.gather(PK, "ragged", BF16, BF16, bs, 8, 128)["kernel"] == tiles
+    assert kernel("ragged", 8, 128, 64) == tiles
+    assert kernel("packed", 3, 128, 256) == tiles
