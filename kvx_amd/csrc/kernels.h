@@ -1821,21 +1821,41 @@ __global__ __launch_bounds__(kBlockThreads) void gather_tiles_kernel(TileArgs a)
     const int32_t lo = tile * region;
     const int64_t valid = ((int64_t)rows << a.cache_es_log2) * re;
     const int32_t hi = (int32_t)(lo + region < valid ? lo + region : valid);
-    for (int32_t m = lo + (int32_t)threadIdx.x * Op::kSrc; m < hi; m += (int32_t)blockDim.x * Op::kSrc) {
-      const uint32_t e = (uint32_t)m >> a.cache_es_log2;
-      int64_t rb = bid;
-      const char *b = blk;
-      if constexpr (FMT == KVX_BLOCK_TABLE_RAGGED) {
-        if (mixed) {
-          rb = s_ids[e / re];
-          if (rb < 0) continue;
-          b = tt.src + rb * tt.s_block;
+    // Chunks of four codes into f32 go four at a time, as in flat_copy: x-packed
+    // K beside NHD V, E5M2 to f32, RAGGED, 16-token blocks, us: 2 x 128, 36000
+    // tokens, 28.1 -> 23.3; 8 x 128, 180000 tokens, 421 -> 364.
+    constexpr int L = flat_unroll<Op>() == kFlatUnrollDequantF32 ? kFlatUnrollDequantF32 : 1;
+    const int32_t step = (int32_t)blockDim.x * Op::kSrc;
+    for (int32_t m0 = lo + (int32_t)threadIdx.x * Op::kSrc; m0 < hi; m0 += L * step) {
+      Raw<Op::kSrc> x[L];
+      float sc[L];
+      bool in[L];
+#pragma unroll
+      for (int u = 0; u < L; ++u) {
+        const int32_t m = m0 + u * step;
+        const uint32_t e = (uint32_t)m >> a.cache_es_log2;
+        int64_t rb = bid;
+        const char *b = blk;
+        in[u] = m < hi;
+        if constexpr (FMT == KVX_BLOCK_TABLE_RAGGED) {
+          if (mixed && in[u]) {
+            rb = s_ids[e / re];
+            in[u] = rb >= 0;
+            b = tt.src + rb * tt.s_block;
+          }
+        }
+        sc[u] = uniform;
+        if (in[u]) {
+          if constexpr (Op::kScaled) sc[u] = scale_in_rows(tt.sc, uniform, rb, e, re, hd);
+          x[u] = ld<Op::kSrc, kGatherNtLoad>(b + part + m);
         }
       }
-      float sc = uniform;
-      if constexpr (Op::kScaled) sc = scale_in_rows(tt.sc, uniform, rb, e, re, hd);
-      st<Op::kDst, kGatherNtStore>(out + ((int64_t)e << a.io_es_log2),
-                                   Op::apply(ld<Op::kSrc, kGatherNtLoad>(b + part + m), sc));
+#pragma unroll
+      for (int u = 0; u < L; ++u) {
+        const uint32_t e = (uint32_t)(m0 + u * step) >> a.cache_es_log2;
+        if (in[u])
+          st<Op::kDst, kGatherNtStore>(out + ((int64_t)e << a.io_es_log2), Op::apply(x[u], sc[u]));
+      }
     }
     return;
   }
