@@ -626,8 +626,14 @@ kvx_status_t enqueue_gather(const GatherPlan &p, void *stream) {
   };
   const bool ragged_tile =
       p.format == KVX_BLOCK_TABLE_RAGGED && rows_contig(p.gk) && rows_contig(p.gv);
+  const bool rows_dense = row_elems_contiguous(p.gk, p.head_dim, p.heads) &&
+                          row_elems_contiguous(p.gv, p.head_dim, p.heads);
+  const bool indexed_f32 = p.conv == kConvDequant && is == 4 && !rows_dense &&
+                           p.format != KVX_BLOCK_TABLE_PACKED &&
+                           row_elems_all < kIndexedDequantF32Row;
   // bytes of cache per chunk at most (FP8: kDequantChunk and its comment)
   const int max_bytes = p.conv != kConvDequant                               ? 16
+                        : indexed_f32                                        ? kDequantChunk
                         : p.format == KVX_BLOCK_TABLE_RAGGED && !ragged_tile && is != 4
                             ? kRaggedDequantChunk
                             : dequant_chunk(is);
@@ -741,11 +747,10 @@ kvx_status_t enqueue_gather(const GatherPlan &p, void *stream) {
     // a multiply-high, exact while tile chunks * nchunks <= 2^32, for rows of
     // at most kFlatRowChunks chunks; otherwise the row kernel, with at least
     // one full pass of its row groups.
-    auto row_dense = [&](const Geom &g) { return row_elems_contiguous(g, p.head_dim, p.heads); };
     const int max_chunks =
         p.conv == kConvDequant && is == 4 ? kFlatRowChunksDequantF32 : kFlatRowChunks;
     const bool chunks_ok = a.nchunks_log2 >= 0 || a.nchunks <= max_chunks;
-    a.flat = row_dense(p.gk) && row_dense(p.gv) && chunks_ok;
+    a.flat = rows_dense && chunks_ok;
     if (ragged_tile && chunks_ok) {
       // R rows of about kFlatTileBytes of cache per tensor: a power of
       // two <= 64 (one block id per lane) that divides block_size

@@ -137,6 +137,13 @@ constexpr int kRaggedDequantChunk = 16;
 // 250 -> 141 / 137 / 143, vLLM's pair PACKED 252 -> 142; HND 128-token blocks
 // RAGGED (16-code chunks before) 197 -> 159.
 constexpr int kDequantChunkF32 = 4;
+// gather_indexed_kernel takes eight into f32 for rows of fewer codes than this,
+// of which four-code chunks leave a wave's lanes or passes half empty.  E5M2 to
+// f32, padded heads, 36000 / 180000 tokens, eight -> four codes, us: 4 x 40
+// RAGGED 17.9 / 89 -> 22.5 / 105, KV_OFFSETS 17.4 / 73 -> 22.8 / 90; 3 x 128
+// KV_OFFSETS 25.4 / 189 -> 28.0 / 199; 4 x 128 RAGGED 31.2 / 240 -> 30.4 / 225,
+// 8 x 128 103 / 493 -> 90 / 419.
+constexpr int64_t kIndexedDequantF32Row = 512;
 // Chunk of a dequantizing gather into io elements of io_size bytes.
 constexpr int dequant_chunk(int io_size) {
   return io_size == 4 ? kDequantChunkF32 : kDequantChunk;
@@ -2422,6 +2429,29 @@ void launch_gather_typed(const GatherArgs &a, int64_t grid, hipStream_t s) {
   }
 }
 
+// gather_indexed_kernel alone (the chunks that only it takes).
+template <class Op>
+void launch_gather_indexed(const GatherArgs &a, int64_t grid, hipStream_t s) {
+  const dim3 g((uint32_t)grid), b(kBlockThreads);
+  constexpr int R = KVX_BLOCK_TABLE_RAGGED, O = KVX_BLOCK_TABLE_KV_OFFSETS;
+  if (a.format == KVX_BLOCK_TABLE_KV_OFFSETS) {
+    if (a.lens_is64)
+      hipLaunchKernelGGL((gather_indexed_kernel<Op, O, true, false>), g, b, 0, s, a);
+    else
+      hipLaunchKernelGGL((gather_indexed_kernel<Op, O, false, false>), g, b, 0, s, a);
+  } else if (a.lens_is64) {
+    if (a.indptr_is64)
+      hipLaunchKernelGGL((gather_indexed_kernel<Op, R, true, true>), g, b, 0, s, a);
+    else
+      hipLaunchKernelGGL((gather_indexed_kernel<Op, R, true, false>), g, b, 0, s, a);
+  } else {
+    if (a.indptr_is64)
+      hipLaunchKernelGGL((gather_indexed_kernel<Op, R, false, true>), g, b, 0, s, a);
+    else
+      hipLaunchKernelGGL((gather_indexed_kernel<Op, R, false, false>), g, b, 0, s, a);
+  }
+}
+
 template <class Op>
 void launch_gather_op(const GatherArgs &a, int64_t grid, hipStream_t s) {
   const bool i64 = a.lens_is64 != 0;  // equals index_is64 for PACKED / RAGGED
@@ -2490,7 +2520,9 @@ void dispatch_quant(int ge, const WriteArgs &a, const WriteLaunch &w, hipStream_
 template <int IO, int F8>
 void dispatch_dequant(int ge, const GatherArgs &a, int64_t grid,
                       hipStream_t s) {
-  if constexpr (IO != KVX_DTYPE_F32) {  // at most kDequantChunkF32 codes there
+  if constexpr (IO == KVX_DTYPE_F32) {  // kDequantChunkF32 codes but there
+    if (ge == 8) return launch_gather_indexed<DequantOp<8, IO, F8>>(a, grid, s);
+  } else {
     if (ge == 16) return launch_gather_op<DequantOp<16, IO, F8>>(a, grid, s);
     if (ge == 8) return launch_gather_op<DequantOp<8, IO, F8>>(a, grid, s);
   }

@@ -76,3 +76,18 @@ def test_copies_of_whole_line_runs_in_big_blocks():
         assert dp.gather(PK, "ragged", BF16, BF16, bs, 8, 128)["kernel"] == tiles
     assert kernel("ragged", 8, 128, 64) == tiles
     assert kernel("packed", 3, 128, 256) == tiles
+
+
+@pytest.mark.parametrize("table", ["ragged", "offsets"])
+def test_short_padded_rows_into_f32_take_chunks_of_eight(table):
+    def chunk(H, D, io=F32, pad=16):
+        plan = dp.gather(NHD, table, E5M2, io, 16, H, D, pad=pad)
+        assert plan["kernel"] == "gather_indexed"
+        return plan["chunk"]
+
+    assert [chunk(H, D) for H, D in ((4, 40), (3, 128), (7, 64))] == [8, 8, 8]
+    assert [chunk(H, D) for H, D in ((4, 128), (8, 128))] == [4, 4]
+    assert chunk(4, 36, pad=12) == 4  # heads that are not whole chunks of eight
+    assert chunk(4, 40, BF16) == 8
+    assert dp.gather(NHD, table, E5M2, F32, 16, 3, 128)["chunk"] == 4  # the flat gathers
+    assert dp.gather(NHD, "packed", E5M2, F32, 16, 3, 128, pad=16)["chunk"] == 4
