@@ -91,3 +91,32 @@ def test_short_padded_rows_into_f32_take_chunks_of_eight(table):
     assert chunk(4, 40, BF16) == 8
     assert dp.gather(NHD, table, E5M2, F32, 16, 3, 128)["chunk"] == 4  # the flat gathers
     assert dp.gather(NHD, "packed", E5M2, F32, 16, 3, 128, pad=16)["chunk"] == 4
+
+
+@pytest.mark.parametrize("bs", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("cache,io", [(BF16, BF16), (F32, F32), (E4M3, BF16), (E5M2, F32)])
+def test_narrow_tiles_hold_whole_units(cache, io, bs):
+    """Tiles of a token-innermost tensor have rows for a whole unit of slots
+    however small the batch, and align on as much as their lanes hold."""
+    seg = 16 // dp.BYTES[cache]
+    for H, D in ((1, 128), (3, 128), (8, 128), (1, 576)):
+        for T in (1, 64, 1000, 4000, 30000):
+            plan = dp.write(dp.VLLM, cache, io, bs, H, D, T, nb=65536)
+            t = plan["t"][1]
+            assert (plan["kernel"], t["kind"]) == ("write_tiles", 2)
+            # at most four runs a thread, with no more than 256 threads
+            runs = t["rows"] * t["tw"] // t["run"]
+            assert plan["threads"] == 256 or plan["threads"] * 4 >= runs
+            assert t["seg"] == seg and t["rows"] == 32
+            align = min(bs, 64 // dp.BYTES[cache], 32)
+            assert t["align"] == align >= seg and t["tw"] >= 32
+
+
+def test_narrow_tiles_that_fill_a_wave():
+    """The shapes that test_gpu_write_tiles.py's WHOLE cases run: 32 rows and 32
+    aligned slots, 16 KiB tiles for the larger copy."""
+    for cache, io, T, tile in ((BF16, BF16, 1100, 4096), (BF16, BF16, 4200, 16384),
+                               (E4M3, BF16, 2100, 4096), (E5M2, F32, 4200, 8192)):
+        for bs in (32, 64, 128):
+            t = dp.write(dp.VLLM, cache, io, bs, 8, 128, T)["t"][1]
+            assert (t["rows"], t["align"], t["rows"] * t["tw"]) == (32, 32, tile)

@@ -130,3 +130,54 @@ def test_row_major_pairs_by_size(fp8, tokens, bs):
     key, val = (torch.randn((s.size, H, D), generator=gen).bfloat16().to(DEV) for _ in range(2))
     check_write(pc, kb, vb, key, val, torch.from_numpy(s).to(DEV), io_dtype=DType.BF16,
                 cache_dtype=dtype, k_scale=0.01 if fp8 else None, v_scale=0.02 if fp8 else None)
+
+
+# (cache, io, tokens) of 8 x 128 rows whose narrow tiles have 32 rows and align
+# on 32 slots, so that all 64 lanes hold slots (test_dispatch_plan.py pins those
+# shapes).  4200 bf16 tokens take 16 KiB tiles.
+WHOLE = [(DType.BF16, DType.BF16, 1100), (DType.BF16, DType.BF16, 4200),
+         (DType.F8_E4M3, DType.BF16, 2100), (DType.F8_E5M2, DType.F32, 4200)]
+
+
+@pytest.mark.parametrize("kind", ["chunks", "spoiled"])
+@pytest.mark.parametrize("bs", [32, 64, 128])
+@pytest.mark.parametrize("cache,io,tokens", WHOLE)
+def test_narrow_tiles_of_32_rows(cache, io, tokens, bs, kind):
+    """vLLM's pair, chunks that start anywhere in a block: units of 16 bytes,
+    runs that a workgroup takes over from its rows, and (spoiled) single runs."""
+    seed = tokens + bs + len(kind)
+    rng = np.random.default_rng(seed)
+    gen = torch.Generator().manual_seed(seed)
+    H, D = 8, 128
+    nb = (2 * tokens + 40 * bs) // bs + 8
+    pc, kb, vb = cache_of("vllm", cache, nb, bs, H, D, gen)
+    s = slots_of(kind, tokens, bs, nb, rng)
+    key, val = ((torch.randn((s.size, H, D), generator=gen) * 2).to(TORCH_DT[io]).to(DEV)
+                for _ in range(2))
+    sc = {}
+    if cache != io and kind == "chunks":
+        sc = dict(k_scale=0.013, v_scale=0.0071)
+    elif cache != io:
+        sc = {f"{t}_scale": ScaleArg(
+            SG.PER_BLOCK_HEAD, torch.empty((nb, H)).uniform_(0.002, 0.05, generator=gen).numpy())
+            for t in "kv"}
+    check_write(pc, kb, vb, key, val, torch.from_numpy(s).to(DEV), io_dtype=io, cache_dtype=cache,
+                **sc)
+
+
+@pytest.mark.parametrize("tokens", [1, 15, 16, 17, 31, 33, 64, 129])
+@pytest.mark.parametrize("start", [0, 1, 15, 40])
+@pytest.mark.parametrize("heads", [1, 3])
+def test_narrow_tiles_of_small_batches(heads, start, tokens):
+    """One chunk into an E4M3 vLLM pair in 64-token blocks: tiles 32 bytes wide
+    whose units start and end inside the rows of one or two workgroups."""
+    gen = torch.Generator().manual_seed(start + tokens)
+    D, bs, nb = 128, 64, 8
+    pc, kb, vb = cache_of("vllm", DType.F8_E4M3, nb, bs, heads, D, gen)
+    ids = torch.randperm(nb, generator=gen)
+    pos = start + torch.arange(tokens)
+    slots = ids[pos // bs] * bs + pos % bs
+    key, val = (torch.randn((tokens, heads, D), generator=gen).bfloat16().to(DEV)
+                for _ in range(2))
+    check_write(pc, kb, vb, key, val, slots.to(DEV), io_dtype=DType.BF16,
+                cache_dtype=DType.F8_E4M3, k_scale=0.01, v_scale=0.02)
