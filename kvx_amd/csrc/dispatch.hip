@@ -393,6 +393,16 @@ constexpr int64_t kWriteDirectWidth = 2048;
 // 13.93 / 46.43; into E4M3 4000 / 10000 / 30000 tokens 7.50 / 14.52 / 34.65
 // -> 7.64 / 12.46 / 34.69; 1 x 576 bf16, 30000 tokens 26.6 -> 24.3; 8 x 256
 // f32, 4000 / 10000 tokens 24.4 / 58.4 -> 21.2 / 60.9.
+// Those are back-to-back writes of the same rows.  Other states of the cache,
+// one write at a time, 19200 tokens of 8 x 128 bf16 and 25600 into E4M3, flat
+// -> tiles: rows just written by another kernel, the rest clean 26.6 -> 28.0
+// and 32.3 -> 28.7, the rest dirty 33.4 -> 27.2 and 34.8 -> 30.8; everything
+// evicted by reads 33.9 -> 34.4 and 36.4 -> 34.2; rows evicted and the cache
+// full of dirty lines, which the rows' allocations then write back, 34.0 ->
+// 46.1 and 36.5 -> 52.0.  A KV write's rows come from the kernel before it, so
+// the last is not tuned for: non-temporal loads take it to 28 and 39, and the
+// back-to-back E4M3 write from 25.4 to 28.3.  Rows of 576 bf16, whose tiles
+// leave a second pass nearly empty, are 5% slower where the rest is clean.
 constexpr int64_t kWriteRowsMin = 12 << 20;
 constexpr int64_t kWriteRowsMax = 256 << 20;
 constexpr int64_t kWriteRowsMinQuant = 32 << 20;
