@@ -1,6 +1,8 @@
 """Build libkvx_amd.so (the C-ABI library with the gfx950 HIP kernels) in-tree.
 
-Usage: python -m kvx_amd.build   (or kvx_amd.build.build() from Python)
+Usage: python -m kvx_amd.build builds everything in this file.  From Python,
+build() makes libkvx_amd.so alone; build_paged_host() makes the module through
+which paged.py builds its descriptors, without which it builds them in ctypes.
 
 Every source is compiled with hipcc for gfx950 only.  Device-code flags:
   -fhip-fp32-correctly-rounded-divide-sqrt  the FP8 quantizing cast divides by

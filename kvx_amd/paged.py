@@ -2,10 +2,10 @@
 
 These build kvx_abi.h descriptors from torch tensors (shape, element strides,
 data pointer, memory type) and call libkvx_amd.so; ``write_kv`` and
-``gather_kv`` have them built natively (csrc/paged_host.cpp).  torch is only
-the source of device memory and streams here; every byte is moved by the
-library's HIP kernels.  There is no fallback: if libkvx_amd.so is missing,
-``abi.load()`` raises.
+``gather_kv`` have them built natively where csrc/paged_host.cpp is built, and
+through ctypes otherwise.  torch is only the source of device memory and
+streams here; every byte is moved by the library's HIP kernels.  There is no
+fallback for those: if libkvx_amd.so is missing, ``abi.load()`` raises.
 
 The calls mirror the reference's launch API (kernels/kvx_paged_kv.h:11-21):
 ``write_kv`` -> kvx_launch_write_kv / kvx_launch_write_kv_prefill,
@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes as C
 import importlib.util
+import warnings
 from dataclasses import dataclass
 from pathlib import Path
 
@@ -25,20 +26,27 @@ from . import abi
 from .abi import DType, Layout, Memory, Status
 
 _HOST_PATH = Path(__file__).resolve().parent / "_paged_host.so"
-_HOST = None
+_HOST = None  # the module, or False where it cannot be loaded
 _STATUS = {int(s): s for s in Status}
 
 
 def _host():
-    """The native descriptor builder (csrc/paged_host.cpp)."""
+    """The native descriptor builder (csrc/paged_host.cpp), or False: it is
+    built for one Python and torch, and where it is missing or made for
+    others the ctypes helpers below build the descriptors."""
     global _HOST
     if _HOST is None:
-        if not _HOST_PATH.exists():
-            raise RuntimeError(f"{_HOST_PATH} is missing; build it with `python -m kvx_amd.build`")
-        spec = importlib.util.spec_from_file_location("_paged_host", _HOST_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        _HOST = module
+        host = False
+        if _HOST_PATH.exists():
+            spec = importlib.util.spec_from_file_location("_paged_host", _HOST_PATH)
+            try:
+                host = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(host)
+            except ImportError as e:
+                host = False
+                warnings.warn(f"{_HOST_PATH.name} does not load ({e}); descriptors are built "
+                              "through ctypes, which takes longer", RuntimeWarning, stacklevel=3)
+        _HOST = host
     return _HOST
 
 
@@ -367,8 +375,9 @@ def write_kv(cache: PagedCache, key: torch.Tensor, value: torch.Tensor,
     name = ("kvx_write_kv" if entry == "abi" else "kvx_launch_write_kv"
             if tokens_per_seq is None else "kvx_launch_write_kv_prefill")
     code = None
-    if type(cache) is PagedCache:
-        code = _host().write(
+    host = _host()
+    if host and type(cache) is PagedCache:
+        code = host.write(
             _address(lib, name), None if entry == "abi" else tokens_per_seq,
             None if stream is None else _stream_handle(stream), *_cache_args(cache), key, value,
             slot_mapping, *_scale_args(k_scale), *_scale_args(v_scale))
@@ -398,7 +407,9 @@ def gather_kv(cache: PagedCache, key_out: torch.Tensor, value_out: torch.Tensor,
     (kvx_launch_gather_kv_dequant).  pool_blocks = (primary, secondary)
     block counts go through kvx_launch_gather_kv_pools instead."""
     lib = abi.load()
-    if type(cache) is PagedCache and pool_blocks is None and (entry != "abi" or k_scale is None):
+    host = _host()
+    if (host and type(cache) is PagedCache and pool_blocks is None
+            and (entry != "abi" or k_scale is None)):
         if isinstance(block_table, RaggedTable):
             table = (block_table.indices, block_table.indptr, None, None, 0)
         elif isinstance(block_table, OffsetsTable):
@@ -408,9 +419,10 @@ def gather_kv(cache: PagedCache, key_out: torch.Tensor, value_out: torch.Tensor,
             table = (block_table, None, None, None, 0)
         name = ("kvx_gather_kv" if entry == "abi" else "kvx_launch_gather_kv"
                 if k_scale is None and v_scale is None else "kvx_launch_gather_kv_dequant")
-        code = _host().gather(
+        code = host.gather(
             _address(lib, name), None if stream is None else _stream_handle(stream),
-            *_cache_args(cache), key_out, value_out, *table, seq_lens, max_seq_len, *_scale_args(k_scale), *_scale_args(v_scale))
+            *_cache_args(cache), key_out, value_out, *table, seq_lens, max_seq_len,
+            *_scale_args(k_scale), *_scale_args(v_scale))
         if code is not None:
             return _STATUS[code]
     # arguments that the native builder leaves to the descriptor helpers

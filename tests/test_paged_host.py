@@ -3,6 +3,7 @@ against the ctypes helpers, on the CPU: over layouts, dtypes, strides, tables
 and scales it hands an entry point the same bytes, and what it does not take
 goes on to the helpers and raises what they raise."""
 import ctypes as C
+import warnings
 
 import pytest
 import torch
@@ -124,3 +125,31 @@ def test_what_the_helpers_refuse_still_raises(entry_points):
         torch.func.vmap(lambda k: paged.write_kv(pc, k, k, slots, stream=STREAM) and k)(
             key[None])
     assert not SEEN
+
+
+@pytest.mark.parametrize("file", ["missing", "of another build"])
+def test_without_the_module_the_helpers_serve(monkeypatch, tmp_path, file):
+    """As before there was one: the library sees the same descriptors."""
+    path = tmp_path / "_paged_host.so"
+    if file != "missing":
+        path.write_bytes(b"not for this Python")
+    monkeypatch.setattr(paged, "_HOST_PATH", path)
+    monkeypatch.setattr(paged, "_HOST", None)
+    lib = abi.bind_like(C.CDLL(str(abi.LIB_PATH)))
+    lib.kvx_launch_write_kv = WRITE
+    lib.kvx_launch_gather_kv = GATHER
+    monkeypatch.setattr(abi, "_LIB", lib)
+    SEEN.clear()
+    pc = next(caches())
+    key = torch.zeros(6, 2, 16, dtype=torch.bfloat16)
+    slots = torch.zeros(6, dtype=torch.int64)
+    with warnings.catch_warnings(record=True) as seen:
+        warnings.simplefilter("always")
+        assert paged.write_kv(pc, key, key, slots, stream=STREAM) == abi.Status.UNSUPPORTED
+        assert SEEN["d"] == bytes(paged.build_write(pc, key, key, slots))
+        out = torch.zeros(3, 16, 2, 16, dtype=torch.bfloat16)
+        table, lens = torch.zeros(3, 4, dtype=torch.int32), torch.zeros(3, dtype=torch.int32)
+        assert paged.gather_kv(pc, out, out, table, lens, 16,
+                               stream=STREAM) == abi.Status.UNSUPPORTED
+        assert SEEN["d"] == bytes(paged.build_gather(out, out, table, lens, 16))
+    assert len(seen) == (file != "missing")
