@@ -173,6 +173,8 @@ def build_paged_host(verbose: bool = False) -> Path:
 
     import torch
 
+    if torch.version.hip is None:
+        raise RuntimeError("the descriptor builder needs a ROCm build of PyTorch")
     tdir = Path(torch.__file__).resolve().parent
     rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)

@@ -8,7 +8,7 @@ import warnings
 import pytest
 import torch
 
-from kvx_amd import abi, paged
+from kvx_amd import abi, build, paged
 from kvx_amd.abi import Layout, ScaleGranularity as SG
 
 SEEN = {}
@@ -153,3 +153,9 @@ def test_without_the_module_the_helpers_serve(monkeypatch, tmp_path, file):
                                stream=STREAM) == abi.Status.UNSUPPORTED
         assert SEEN["d"] == bytes(paged.build_gather(out, out, table, lens, 16))
     assert len(seen) == (file != "missing")
+
+
+def test_build_without_rocm_says_so(monkeypatch):
+    monkeypatch.setattr(torch.version, "hip", None)
+    with pytest.raises(RuntimeError, match="ROCm build of PyTorch"):
+        build.build_paged_host()
