@@ -120,3 +120,27 @@ def test_narrow_tiles_that_fill_a_wave():
         for bs in (32, 64, 128):
             t = dp.write(dp.VLLM, cache, io, bs, 8, 128, T)["t"][1]
             assert (t["rows"], t["align"], t["rows"] * t["tw"]) == (32, 32, tile)
+
+
+def test_quantizing_writes_by_chunk():
+    """The kernels and chunks that test_gpu_fp8_paths.py's CHUNKS cases run."""
+    for H, D, pad, codes in ((4, 64, 8, 8), (4, 64, 4, 4), (4, 64, 2, 2), (4, 64, 1, 1),
+                             (4, 40, 0, 8), (4, 12, 0, 4), (3, 6, 0, 2), (3, 7, 0, 1)):
+        for io in (BF16, DType.F16, F32):
+            for bs in (16, 20):
+                plan = dp.write(HND, E4M3, io, bs, H, D, 90, pad=pad)
+                assert (plan["kernel"], plan["chunk"]) == ("write", codes)
+                plan = dp.write(NHD, E4M3, io, bs, H, D, 90, pad=pad)
+                assert plan["chunk"] == codes
+                assert plan["kernel"] == ("write" if pad else "write_flat")
+
+
+def test_ragged_tiles_of_sparse_batches():
+    """The rows per tile that test_gpu_gather_skew.py's cases run."""
+    for cache, io, H, D, base in ((BF16, BF16, 1, 776, 1), (E4M3, BF16, 2, 776, 1),
+                                  (E5M2, F32, 1, 1552, 1), (BF16, BF16, 1, 392, 2),
+                                  (BF16, BF16, 1, 576, 2)):
+        full = base * 49152
+        for entries, r in ((full - 1, base), (full, 2 * base)):
+            plan = dp.gather(NHD, "ragged", cache, io, 16, H, D, S=24, L=full, entries=entries)
+            assert (plan["kernel"], plan["rows"]) == ("gather_ragged_tile", r)

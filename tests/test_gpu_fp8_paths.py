@@ -1,10 +1,13 @@
 """GPU parity of the FP8 casts on the kernel paths that only some shapes
 reach, through the C ABI, bit-identical to the CPU oracle:
 
-  write_kernel with the quantizing op   a decode write (fewer tokens than
-      block_size, so no whole block for the tiled write) into caches whose
-      rows are not contiguous: HND, x-packed, and vLLM's value cache
-      [num_blocks, H, D, block_size] (CUSTOM);
+  write_kernel with the quantizing op   caches padded inside a block and
+      heads that are not whole chunks, in chunks of 8, 4, 2 and 1 codes;
+  write_flat_kernel with the quantizing op   row-major caches of such heads;
+  write_tiles_kernel with the quantizing op   a decode write (fewer tokens
+      than block_size) into caches whose rows are not contiguous: HND,
+      x-packed, and vLLM's value cache [num_blocks, H, D, block_size]
+      (CUSTOM);
   gather_rows_kernel with the dequantizing op   PACKED gathers of HND
       caches whose heads are 40 FP8 bytes (runs the LDS tile kernel cannot
       cut into 16-byte pieces);
@@ -24,7 +27,7 @@ import torch
 from kvx_amd import paged
 from kvx_amd.abi import DType, Layout, ScaleGranularity as SG
 
-from gpu_helpers import (TORCH_DT, OffsetsPool, ScaleArg, check_gather, check_gather_offsets,
+from gpu_helpers import (TORCH_DT, CacheBuf, OffsetsPool, ScaleArg, check_gather, check_gather_offsets,
                          check_gather_ragged, check_write, custom_cache, make_cache,
                          random_fill)
 
@@ -59,7 +62,7 @@ def scales(kind, gen, nb, H):
 @pytest.mark.parametrize("layout", ["hnd", "packed", "vllm_v"])
 def test_quantizing_decode_write_token_path(layout, fp8, kind):
     gen = torch.Generator().manual_seed(50 + KINDS.index(kind) + 4 * FP8.index(fp8))
-    H, D, bs, nb, T = 8, 128, 16, 40, 11  # T < bs: no whole block
+    H, D, bs, nb, T = 8, 128, 16, 40, 11  # T < bs
     if layout == "vllm_v":
         pc, kb, vb = custom_cache(fp8, nb, bs, H, D, "bhdo", "bhdo", gen=gen)
     else:
@@ -69,6 +72,38 @@ def test_quantizing_decode_write_token_path(layout, fp8, kind):
     key, val = rows(T, H, D, io, gen, 2.0), rows(T, H, D, io, gen, 0.3)
     slots = torch.randperm(nb * bs, generator=gen)[:T]
     slots[3] = -1
+    ks, vs = scales(kind, gen, nb, H)
+    check_write(pc, kb, vb, key, val, slots.to(DEV), io_dtype=io, cache_dtype=fp8,
+                k_scale=ks, v_scale=vs)
+
+
+# (H, D, elements of padding after each head run, codes per chunk): padded
+# heads and HND take write_kernel, NHD ones write_flat_kernel
+# (test_dispatch_plan.py pins both)
+CHUNKS = [(4, 64, 8, 8), (4, 64, 4, 4), (4, 64, 2, 2), (4, 64, 1, 1), (4, 40, 0, 8),
+          (4, 12, 0, 4), (3, 6, 0, 2), (3, 7, 0, 1)]
+
+
+@pytest.mark.parametrize("kind", ["tensor", "block_head"])
+@pytest.mark.parametrize("fp8", FP8)
+@pytest.mark.parametrize("layout", [NHD, HND])
+@pytest.mark.parametrize("shape", CHUNKS)
+def test_quantizing_write_by_chunk(shape, layout, fp8, kind):
+    H, D, pad, _ = shape
+    case = CHUNKS.index(shape) + FP8.index(fp8) + (kind == "tensor")
+    gen = torch.Generator().manual_seed(90 + 4 * case + int(layout))
+    bs, nb, T = [16, 20][case % 2], 12, 90
+    io = [DType.BF16, DType.F16, DType.F32][case % 3]
+    kb, vb = (CacheBuf(layout, fp8, nb, bs, H, D, 8, DEV, gen, 3 if pad else None, pad)
+              for _ in range(2))
+    pc = paged.PagedCache(kb.view, vb.view, layout, layout, nb, bs, H, D)
+    key, val = rows(T, H, D, io, gen, 2.0), rows(T, H, D, io, gen, 0.3)
+    key.view(-1)[::37] = float("nan")
+    val.view(-1)[::41] = float("inf")
+    slots = torch.randperm(nb * bs, generator=gen)[:T]
+    slots[3], slots[50] = -1, nb * bs + 3
+    if case % 2:
+        slots = slots.to(torch.int32)
     ks, vs = scales(kind, gen, nb, H)
     check_write(pc, kb, vb, key, val, slots.to(DEV), io_dtype=io, cache_dtype=fp8,
                 k_scale=ks, v_scale=vs)

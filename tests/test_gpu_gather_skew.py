@@ -6,9 +6,9 @@ import pytest
 import torch
 
 from kvx_amd import paged
-from kvx_amd.abi import DType, Layout
+from kvx_amd.abi import DType, Layout, ScaleGranularity as SG
 
-from gpu_helpers import (TORCH_DT, OffsetsPool, check_gather, check_gather_offsets,
+from gpu_helpers import (TORCH_DT, OffsetsPool, ScaleArg, check_gather, check_gather_offsets,
                          check_gather_ragged, make_cache, random_fill)
 
 pytestmark = pytest.mark.gpu
@@ -44,6 +44,40 @@ def test_ragged_sparse_tiles(extra):
     dl[0], dl[1], dl[2], dl[4] = 0, -3, 77, L + 9
     check_gather_ragged(pc, kb, vb, ko, vo, table, torch.from_numpy(dl.astype(np.int32)).to(DEV),
                         L, cache_dtype=DType.BF16, io_dtype=DType.BF16)
+
+
+@pytest.mark.parametrize("cache,io,H,D,base", [(DType.BF16, DType.BF16, 1, 392, 2),
+                                               (DType.F8_E4M3, DType.BF16, 2, 776, 1),
+                                               (DType.F8_E5M2, DType.F32, 1, 1552, 1)])
+def test_ragged_sparse_tiles_of_other_rows(cache, io, H, D, base):
+    """The rule in effect on tiles of two rows (four), and on FP8 rows with
+    per-block-head scales: whole blocks and rows of a tile in several blocks."""
+    rng = np.random.default_rng(D)
+    gen = torch.Generator().manual_seed(D)
+    bs, S, total = 16, 24, base * 49152
+    L = 3 * total // S + 33
+    lens = np.full(S, L)
+    lens[7:] = (total - 7 * L) // (S - 7)
+    lens[-1] += total - lens.sum()
+    assert lens.sum() == total and lens.max() == L and total * 3 < S * L
+    nb = 500
+    pc, kb, vb = make_cache(NHD, NHD, cache, nb, bs, H, D, gen=gen)
+    rows = [np.repeat(rng.integers(0, nb, size=-(-n // bs)), bs)[:n] for n in lens]
+    rows[3][::7] = nb - 2
+    rows[9][::3] = -1
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    table = paged.RaggedTable(torch.from_numpy(np.concatenate(rows).astype(np.int32)).to(DEV),
+                              torch.from_numpy(indptr).to(DEV))
+    sc = {}
+    if cache != io:
+        sc = {f"{t}_scale": ScaleArg(SG.PER_BLOCK_HEAD, rng.uniform(0.01, 0.05, (nb, H)))
+              for t in "kv"}
+    ko = torch.zeros((S, L, H, D), dtype=TORCH_DT[io], device=DEV)
+    vo = torch.zeros_like(ko)
+    dl = lens.copy()
+    dl[0], dl[1], dl[8] = 77, L + 9, 0
+    check_gather_ragged(pc, kb, vb, ko, vo, table, torch.from_numpy(dl.astype(np.int32)).to(DEV),
+                        L, cache_dtype=cache, io_dtype=io, **sc)
 
 
 @pytest.mark.parametrize("fp8", [False, True])
