@@ -863,8 +863,8 @@ __global__ __launch_bounds__(kBlockThreads) void write_tiles_kernel(WriteTileArg
       x[k] = ld<Op::kSrc, kWriteNtLoad>(src + row[k] * a.row_bytes +
                                         (int64_t)(u - row[k] * t.cpr) * Op::kSrc);
   }
-  // Lane l holds the slot of row l - lane0 of the tile (narrow: from the row
-  // before it to the rows that may follow it).  Loaded behind the rows, whose
+  // Lane l holds the slot of row l - lane0 of the tile (align > 1, staged or
+  // narrow: lane0 = 1, from the row before it to the rows that may follow it).  Loaded behind the rows, whose
   // addresses do not need it: 32768 tokens of 8 x 128 bf16 into x-packed K
   // and NHD V 53.7 -> 53.1 us.
   const int64_t ts = t0 + lane - lane0;
@@ -1518,7 +1518,7 @@ struct TileArgs {
   int32_t cpr;            // tw_log2 < 0: phase-2 chunks per tile row
   uint32_t cpr_magic;     // tw_log2 < 0: div_magic's m for cpr
   int32_t pitch;          // LDS row pitch, bytes
-  int32_t threads;        // workgroup size (128 for small tiles, else 256)
+  int32_t threads;        // workgroup size, 64 to 256
   int32_t max_seq_len;
   int32_t num_blocks;
   int32_t head_dim;

@@ -7,12 +7,11 @@ stores a row as H * D consecutive elements and takes the row-major kernels (writ
 and KV_OFFSETS flat gathers), for copies and FP8 casts.
 
 Blocks of 128 and 256 tokens take paths that smaller ones do not:
-  gather_rows_kernel   a block's rows split over several workgroups (HND
-      rows whose 64 KiB tile does not fit LDS, padded blocks, FP8 heads of
-      40 bytes with the dequantizing op), parts that start past seq_len,
-      parts cut by seq_len, and ids < 0 or >= num_blocks;
-  gather_tiles_kernel  tiles of one 128-byte line per row (x-packed and
-      token-innermost blocks, 16 and 32 KiB tiles) and 32 KiB HND tiles.
+  gather_rows_kernel   a block's rows split over several workgroups (padded
+      blocks, FP8 heads of 40 bytes with the dequantizing op), parts that
+      start past seq_len, parts cut by seq_len, and ids < 0 or >= num_blocks;
+  gather_tiles_kernel  parts of 64 rows of a block (x-packed, token-innermost
+      and, where the flat gather's head runs do not apply, HND blocks).
 """
 import pytest
 import torch
@@ -32,8 +31,8 @@ DEV = "cuda"
 
 # (cache dtype, K order, K x, V order, V x, block_size, H, D, pad)
 CASES = [
-    (DType.BF16, "bhod", None, "bhod", None, 256, 8, 128, 0),   # HND: row kernel, split
-    (DType.BF16, "bhod", None, "bhod", None, 128, 8, 128, 0),   # HND: 32 KiB tiles
+    (DType.BF16, "bhod", None, "bhod", None, 256, 8, 128, 0),   # HND: flat, head runs
+    (DType.BF16, "bhod", None, "bhod", None, 128, 8, 128, 0),   # the same
     (DType.BF16, "bhpox", 8, "bohd", None, 256, 8, 128, 0),     # x-packed: 128-byte tiles
     (DType.BF16, "bhdo", None, "bhpox", 8, 128, 8, 128, 0),     # token-innermost / x-packed
     (DType.F16, "obhd", None, "hbod", None, 128, 4, 64, 1),     # padded: row kernel, split
@@ -261,9 +260,8 @@ def test_head_run_flat_gather(case, idx64):
                  cache_dtype=dt, io_dtype=io, k_scale=ks, v_scale=vs)
 
 
-# RAGGED gathers of dense blocks of more than 64 tokens in the LDS tiles:
-# every thread loads row ids, and one barrier tells whether a tile names one
-# block.  (cache dtype, K order, K x, V order, V x, block_size, H, D)
+# RAGGED gathers of dense blocks of more than 64 tokens, in the LDS tiles in
+# parts of 64 rows, whose ids one wave loads.  (cache dtype, K order, K x, V order, V x, block_size, H, D)
 RAGGED_BIG = [
     (DType.BF16, "bhpox", 8, "bohd", None, 128, 8, 128),     # x-packed K, NHD V
     (DType.BF16, "bhpox", 8, "bhdo", None, 256, 4, 64),      # vLLM's pair

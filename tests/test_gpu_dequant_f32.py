@@ -18,12 +18,13 @@ NHD, HND, PK = Layout.BLOCK_NHD, Layout.BLOCK_HND, Layout.BLOCK_HND_PACKED
 
 
 @pytest.mark.parametrize("table", ["packed", "ragged", "offsets"])
-@pytest.mark.parametrize("layout", [NHD, HND, PK])
-@pytest.mark.parametrize("shape", [(8, 128), (4, 12), (4, 36), (1, 576), (3, 7), (2, 16)])
+@pytest.mark.parametrize("shape,layout", [
+    (shape, layout)
+    for shape in ((8, 128), (4, 12), (4, 36), (1, 576), (3, 7), (2, 16))
+    for layout in (NHD, HND, PK)
+    if not (layout == PK and shape[1] % 4)])  # packs of 4
 def test_gather_into_f32(shape, layout, table):
     H, D = shape
-    if layout == PK and D % 4:
-        pytest.skip("packs of 4")
     seed = H * 1000 + D + 7 * int(layout)
     rng = np.random.default_rng(seed)
     gen = torch.Generator().manual_seed(seed)

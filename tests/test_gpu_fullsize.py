@@ -377,8 +377,7 @@ WRITE_SHAPES = [  # (name, layouts, heads, head_dim, block_size)
 @pytest.mark.parametrize("shape", WRITE_SHAPES, ids=[c[0] for c in WRITE_SHAPES])
 def test_c3_full_other_shapes(shape):
     """c3's prefill chunks into caches of other rows and block sizes (tiles
-    of whole runs, the per-token path of 128-token blocks, one-token
-    blocks): every written row in place, untouched blocks unchanged, and the
+    of whole runs, blocks of 128 tokens, one-token blocks): every written row in place, untouched blocks unchanged, and the
     gather returning the input rows."""
     _, lay, H, D, bs = shape
     w = workloads.c3_llama8b_prefill(block_size=bs)
@@ -485,10 +484,9 @@ def test_flat_write_rows_not_pow2_chunks():
 def test_c3_size_chunks_starting_inside_blocks(layout):
     """c3's size (16 sequences x 2048 tokens) with every chunk starting at a
     different offset inside its first block, into x-packed K with NHD V or
-    vLLM's pair (x-packed K, token-innermost V): each block is owned by the
-    group where its run starts (whole-block and shifted fast paths, the
-    two-run groups at chunk starts).  Every row must land at its slot, every
-    other byte of the caches keep its value."""
+    vLLM's pair (x-packed K, token-innermost V): tokens of one line of a run
+    belong to the workgroup in whose rows they start.  Every row must land at
+    its slot, every other byte of the caches keep its value."""
     H, D, bs, S, C, nb = 8, 128, 16, 16, 2048, 8192
     gen = torch.Generator().manual_seed(81)
     perm = torch.randperm(nb, generator=gen)

@@ -223,10 +223,10 @@ def test_fp8_write_and_dequant_gather_graph_replays(gran):
 
 def test_prefill_tile_write_graph_replays():
     """The tiled prefill write (K x-packed, V NHD, whole-block chunks)
-    captured once.  Later replays spoil some groups (-1 slots, swapped
-    offsets, a chunk shifted inside its block), which the kernels route to
-    the per-token and two-run paths on the device: the captured launch is
-    the same for every slot pattern."""
+    captured once.  Later replays spoil some blocks (-1 slots, swapped
+    offsets, a chunk shifted inside its block): which tokens a workgroup stores,
+    and how, is decided on the device, so the captured launch is the same for
+    every slot pattern."""
     gen = torch.Generator().manual_seed(9)
     rng = np.random.default_rng(21)
     nb, bs, H, D = 64, 16, 8, 128

@@ -1,5 +1,5 @@
 """GPU parity of the LDS tile kernels: the transposing gather
-(gather_tiles_kernel) and the tiled block write (write_tiles_kernel), for
+(gather_tiles_kernel) and the tiled write (write_tiles_kernel), for
 dense blocks that are not row-major — token axis innermost (vLLM's value
 cache [num_blocks, H, D, block_size]), x-packed HND_PACKED, HND — through
 the C ABI, bit-identical to the CPU oracle (kernels/kvx_paged_kv.cu:93-124
@@ -13,10 +13,11 @@ of 96 or 80 elements, rows of 3 or 6 heads), a row-major partner tensor, partial
 FP8 dequantizing gather with per-tensor, per-head and per-block-head
 scales.  RAGGED cases cover tiles whose rows all name one block, tiles whose
 rows name different blocks or invalid ones, short indptr ranges and int64
-indptr.  Write cases cover the same layouts with groups that fill a block
-in order, groups that do not (partial, out of order, invalid slots, a
-ragged tail), and the quantizing FP8 write, also with tile widths that are
-not a power of two.
+indptr.  Write cases cover the same layouts (direct, staged and narrow
+tensors) with blocks filled in order, chunks that start inside blocks, so that
+tokens go on with a line or unit of the previous workgroup's rows, tokens out
+of order or without a slot, a ragged tail, and the quantizing FP8 write, also
+with tile widths that are not a power of two.
 """
 import numpy as np
 import pytest
@@ -130,7 +131,8 @@ def test_tiles_hnd_packed_layouts(entry):
 def _prefill_slots(gen, nb, bs, groups, tail, spoil):
     """Slots of `groups` full blocks in order (random distinct blocks), then
     `tail` tokens; `spoil` groups get one slot changed (-1, a swap, or a
-    block past the end) so that they take the per-token path."""
+    block past the end): the rest of its tokens still go to their slots, in
+    narrow tensors run by run."""
     blocks = torch.randperm(nb, generator=gen)[: groups + 1]
     slots = (blocks[:groups, None] * bs + torch.arange(bs)).reshape(-1)
     slots = torch.cat([slots, blocks[groups] * bs + torch.arange(tail)])
@@ -166,8 +168,7 @@ def test_tiles_write(case, slot64):
 @pytest.mark.parametrize("io", [DType.BF16, DType.F16, DType.F32])
 def test_tiles_quantizing_write(fp8, io):
     """K token-innermost, V x-packed x = 16: the tile op quantizes 8
-    elements per chunk; per-tensor scales (indexed scales use the per-token
-    kernel)."""
+    elements per chunk; per-tensor scales."""
     gen = torch.Generator().manual_seed(300 + int(fp8) * 10 + int(io))
     H, D, bs, nb = 8, 128, 16, 40
     pc, kb, vb = custom_cache(fp8, nb, bs, H, D, "bhdo", "bhpox", None, 16, gen)
@@ -197,8 +198,8 @@ def test_tiles_write_x_packed_entries(entry):
 
 
 def _whole_block_edge_slots(gen, nb, bs, slot64):
-    """Groups aimed at the whole-block test of the tiled write: in order in
-    the block past the end (skipped), in the last and the first block, in
+    """Blocks' worth of tokens at the edges of the tiled write's slots: in
+    order in the block past the end (skipped), in the last and the first block, in
     reverse order, one slot repeated, and for int64 slots an in-order group
     at 2**32 (its block id needs the slot's high word); ordinary whole
     blocks in between."""
@@ -222,9 +223,10 @@ def _whole_block_edge_slots(gen, nb, bs, slot64):
                          ids=[_ids(c) for c in (CASES[0], CASES[2], CASES[3])])
 @pytest.mark.parametrize("slot64", [False, True])
 def test_tiles_write_whole_block_edges(case, slot64):
-    """The whole-block path of write_tiles_kernel takes a group only when its
-    slots are block * bs + 0 .. bs - 1 in token order with block < num_blocks;
-    every other group falls back to the run analysis or the per-token path."""
+    """Tokens of one block in order are stored as whole units and pieces of
+    consecutive slots, those in other orders one by one, those past the blocks
+    not at all; a slot named twice ends with its last token's row, as in the
+    oracle."""
     dt, ko_, kx, vo_, vx, bs, H, D = case
     gen = torch.Generator().manual_seed(330 + CASES.index(case) * 2 + int(slot64))
     nb = 24
@@ -266,9 +268,9 @@ def _unaligned_chunk_slots(gen, nb, bs, seqs, spoil):
 @pytest.mark.parametrize("case", CASES, ids=[_ids(c) for c in CASES])
 @pytest.mark.parametrize("spoil", [0, 3])
 def test_tiles_write_unaligned_chunks(case, spoil):
-    """Chunks that start inside blocks: each block's run is owned by the
-    workgroups of the group where the run starts, and runs cross group and
-    sequence boundaries."""
+    """Chunks that start inside blocks: tokens of one line (narrow: sector) of
+    a run belong to the workgroup in whose rows they start, across workgroups
+    and sequences."""
     dt, ko_, kx, vo_, vx, bs, H, D = case
     gen = torch.Generator().manual_seed(340 + CASES.index(case) * 2 + int(spoil > 0))
     nb = 96
@@ -374,9 +376,9 @@ def test_tiles_write_chunks_inside_blocks(case):
 @pytest.mark.parametrize("case", [c for c in CASES if c[5] >= 4],
                          ids=[_ids(c) for c in CASES if c[5] >= 4])
 def test_tiles_write_two_runs(case):
-    """Full groups of two runs in different blocks (the tail of one block
-    from offset 3, the head of another from offset 2), then a last, short
-    group of two runs inside one block around a gap (offsets [1, bs/2) and
+    """Blocks' worth of tokens in two runs in different blocks (the tail of one
+    block from offset 3, the head of another from offset 2), then fewer in two
+    runs inside one block around a gap (offsets [1, bs/2) and
     [bs/2 + 1, bs): rows 0 and bs/2 keep their contents)."""
     dt, ko_, kx, vo_, vx, bs, H, D = case
     gen = torch.Generator().manual_seed(550 + CASES.index(case))
@@ -414,8 +416,8 @@ def test_tiles_quantizing_write_chunks(fp8):
 @pytest.mark.parametrize("layouts", [("bhdo", None, "bhpox", 16), ("bhpox", 16, "bohd", None)])
 def test_tiles_quantizing_write_indexed_scales(kind, layouts):
     """Indexed scales through the tiled write: whole blocks, chunks that
-    start inside blocks (the scale follows each run's block) and spoiled
-    groups (per-token path)."""
+    start inside blocks (the scale follows each token's block) and spoiled
+    blocks."""
     ko_, kx, vo_, vx = layouts
     gen = torch.Generator().manual_seed(600 + int(kind) * 3 + (kx is None))
     H, D, bs, nb = 8, 128, 16, 64
@@ -455,7 +457,7 @@ def test_tiles_quantizing_write_indexed_scales(kind, layouts):
 def test_tiles_quantizing_write_odd_tiles(shape, fp8, kind):
     """The quantizing tiled write with tile widths that are not a power of
     two (96- and 80-byte FP8 runs, 384-byte rows): whole blocks, spoiled
-    groups and chunks that start inside blocks."""
+    ones and chunks that start inside blocks."""
     ko_, kx, vo_, vx, H, D = shape
     gen = torch.Generator().manual_seed(700 + 4 * H + int(fp8) + 2 * (kind != "tensor"))
     bs, nb = 16, 64
@@ -485,9 +487,9 @@ _ROW_MAJOR_PAIRS = [("bohd", None, "bhpox", 8), ("bhpox", 8, "bohd", None),
 @pytest.mark.parametrize("seed", range(15))
 def test_tiles_write_row_major_ownership(seed):
     """Seeded prefill chunks (random starts inside blocks, random lengths,
-    spoiled slots, both write entries) into caches where a row-major tensor
-    is written group by group, its own tokens only, beside a partner whose
-    runs belong to the group they start in: the whole cache must equal the
+    spoiled slots, both write entries) into caches where a row-major tensor's
+    workgroups write their own tokens only, beside a partner's whose tokens may
+    belong to the workgroup before: the whole cache must equal the
     oracle's, every untouched byte included."""
     rng = np.random.default_rng(900 + seed)
     gen = torch.Generator().manual_seed(900 + seed)
@@ -518,8 +520,8 @@ def test_tiles_decode_write_mixed_layouts(layouts, dt):
     """A decode batch (one new token per sequence, each in a block of its
     own, at any offset; some slots -1 or past the pool) into K / V pairs of
     different piece sizes (16-byte x-packed or HND pieces beside one-element
-    token-innermost ones): write_tiles_kernel's groups fill no block, so
-    every token goes through its per-token fallback."""
+    token-innermost ones): no two tokens share a unit, so narrow tensors store
+    every token run by run."""
     ko_, kx, vo_, vx = layouts
     gen = torch.Generator().manual_seed(520 + int(dt) * 8 + ["bhpox", "bhdo", "bhod"].index(ko_))
     H, D, bs, nb, T = 8, 128, 16, 96, 70

@@ -82,11 +82,8 @@ def tables():
         yield paged.OffsetsTable(torch.zeros(3, 1, 2, 4, dtype=torch.int32), pool, sec, 256)
 
 
-@pytest.mark.parametrize("scale", SCALES)
-@pytest.mark.parametrize("entry", ["launch", "abi"])
+@pytest.mark.parametrize("scale,entry", [(s, "launch") for s in SCALES] + [(None, "abi")])
 def test_gather_descriptors(entry_points, scale, entry):
-    if entry == "abi" and scale is not None:
-        pytest.skip("kvx_gather_kv takes no scales")
     for pc in caches():
         for tb in tables():
             ko = torch.zeros(3, 16, 2, 16, dtype=torch.float16)
