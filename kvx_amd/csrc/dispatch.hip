@@ -419,13 +419,10 @@ int64_t tile_width(int64_t row, int64_t unit, int64_t target) {
     return w;
   }
   int64_t best = -1, line = -1;
-  for (int64_t k = 1; k <= row / unit; ++k) {
-    if ((row / unit) % k != 0) continue;
-    const int64_t w = unit * k;
-    if (w > target && best > 0) break;
-    best = w;
-    if (w % 128 == 0) line = w;
-    if (w > target) break;
+  for (int64_t k = 1; k <= n && (best < 0 || unit * k <= target); ++k) {
+    if (n % k != 0) continue;
+    best = unit * k;
+    if (best % 128 == 0) line = best;
   }
   return line > 0 ? line : best;
 }
