@@ -367,17 +367,17 @@ constexpr int64_t kWriteTileWorkgroups = 512;
 // against 33) and x-packed chunks that start inside blocks took 38 against
 // 27; 64 leave a wave no lanes for the rows that follow (narrow: 174).
 constexpr int64_t kWriteTileRows = 32;
-// Cache bytes per row of a staged and of a narrow tensor's workgroup, at least,
-// where small batches make small tiles: a narrow one keeps kWriteTileRows rows,
-// since a unit is 16 bytes of consecutive slots (16 rows of FP8 codes), and has
-// a thread for every kTileLoads runs, since decode batches store it one run at
-// a time.  vLLM's pair, us, 128-byte rows and threads by bytes -> now: E4M3, 4000
-// tokens of 1 x 128 in 64 / 128-token blocks 27.4 / 42 -> 6.0 / 6.3, 1000 of 3 x
-// 128 23 / 28 -> 6.5 / 6.7, 64 decode tokens of 8 x 128 in 16-token blocks 6.6 ->
-// 5.6, 8 tokens 6.1 -> 5.3; bf16, 1000 tokens, 11% over heads and blocks; f32
-// unchanged.
+// Cache bytes per row of a workgroup through LDS, at least, where small batches
+// make small tiles: kWriteStagedWidth, or kWriteNarrowRuns narrow runs where
+// those are fewer bytes, so that a tile's rows hold whole units (16 rows of FP8
+// codes).  Narrow tensors also have a thread for every kTileLoads runs, since
+// decode batches store one run at a time.  vLLM's pair, us, 128-byte rows and
+// threads by bytes -> now: E4M3, 4000 tokens of 1 x 128 in 64 / 128-token blocks
+// 27.4 / 42 -> 6.0 / 6.3, 1000 of 3 x 128 23 / 28 -> 6.5 / 6.7, 64 decode tokens
+// of 8 x 128 in 16-token blocks 6.6 -> 5.6, 8 tokens 6.1 -> 5.3; bf16, 1000
+// tokens, 7% over heads and blocks; f32 the same.
 constexpr int64_t kWriteStagedWidth = 128;
-constexpr int64_t kWriteNarrowWidth = 32;
+constexpr int64_t kWriteNarrowRuns = 32;
 // Bytes of a narrow run that one workgroup stores whole, at most.
 constexpr int64_t kWriteAlignBytes = 64;
 // Bytes per row of a direct tensor's workgroup, at most: whole rows of 2 KiB
@@ -472,7 +472,9 @@ bool plan_write_tiles(const WritePlan &p, int cs, int is, WriteTileArgs *wt, int
       tile = kWriteLdsCopyBytes;
     // a tile holds whole 16-byte pieces and whole runs
     const int64_t unit = w == H * D || run < 16 ? 16 : run;
-    const int64_t least = t.kind == kTileNarrow ? kWriteNarrowWidth : kWriteStagedWidth;
+    const int64_t least = t.kind == kTileNarrow && kWriteNarrowRuns * run < kWriteStagedWidth
+                              ? kWriteNarrowRuns * run
+                              : kWriteStagedWidth;
     const int64_t target = t.kind == kTileDirect
                                ? (tile < kWriteDirectWidth ? tile : kWriteDirectWidth)
                                : (tile / kWriteTileRows < least ? least : tile / kWriteTileRows);
